@@ -703,7 +703,8 @@ struct Sched {
   }
   // after the sync of a trial rotation: charge its time, decide when done
   void trial_sample() {
-    if (trials.empty()) return;
+    dirty = true;  // a trial chunk has no graph: the next chunk lists its own
+    if (trials.empty()) return;  // the class on trial left with its last set
     Trial& t = trials.front();
     if (t.timed && t.units > 0.0) {
       float ms = 0.0f;
@@ -735,7 +736,6 @@ struct Sched {
                      t.cand[best]);
       trials.pop_front();
     }
-    dirty = true;
   }
   int n_tiles_s = 0, n_tiles_c = 0, n_ids = 0;
   // Fast lane: sets at most 1/8 the size (columns) of the largest resident

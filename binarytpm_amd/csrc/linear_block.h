@@ -1,0 +1,245 @@
+// linear_block.h -- eight explicit conduction steps of a column as one matrix
+// product on the matrix cores.
+//
+// Between two surface balances the explicit step is linear in the 55 interior
+// nodes, so the nodes after the 8 steps of a time block are
+//     nodes' = P^8 nodes + sum_j H_j u0(j),     j = 0..7,
+// with u0(j) the surface offset before step j of the block, and node 1, the
+// only node the surface balance of a step reads, is after s steps
+//     u1(s) = base(s) + sum_{j < s} g(s-1-j) u0(j),
+// base(s) being the part due to the nodes at the block's start.  base(1..8)
+// of the NEXT block is again linear in (nodes, u0(0..7)), so one 64 x 64
+// product per block gives both: 55 nodes + 8 surface values in, 55 nodes + 8
+// responses out (one spare).  A step then costs the surface balance and at
+// most 8 FMAs (36 a block) instead of 110 vector instructions.
+//
+// Layout.  The product runs on v_mfma_f32_16x16x32_f16: lane l supplies
+// A[m = l%16][k = 8(l/16)+j] and B[k = 8(l/16)+j][n = l%16], j < 8, and
+// receives D[m = 4(l/16)+i][n = l%16], i < 4.  A tile of 16 columns is held
+// as u[16] per lane, lane (g = l/16, c = l%16) the 16 slots q of group g of
+// column c.  Slot (g, q) is row 4(q/4).. of output tile t = q/4 and K entry of
+// input chunk h = q/8, so the product's output is the next product's input
+// without moving between lanes.  Which node a slot holds is free; with
+//     tile 0: q = 0, 1: u0(2g + q) in, base(2g + q + 1) out;
+//             q = 2, 3: node 1 + 2g + (q - 2)
+//     tile t > 0:       node 9 + 16(t-1) + 4g + (q - 4t)
+// the 17-wide band of P^8 leaves the blocks (tile 0, chunk 1) and (tile 3,
+// chunk 0) empty: 6 of 8 blocks are stored and multiplied.
+//
+// Precision.  Operator and columns are split x = hi + lo in fp16 and
+// multiplied as lo hi + hi lo + hi hi with FP32 accumulation.  A column value
+// is FP32 (24 bits) and fp16 holds 11, so hi + lo (rounded to nearest) drops
+// at most one unit of the last FP32 place; the operator is scaled by 2^15 so
+// that its low halves stay normal numbers, and the rounding of its low halves
+// is carried along each row, so that constants stay constants to 2^-24 of an
+// ulp.  Columns are held multiplied by 2^15 (as the product leaves them).
+// Against FP64 over 24 to 60 rotations (r 0.03..0.497, inertias 30..2000) the
+// surface temperatures are within 6.3-7.5e-6 K rms, where eight FP32 steps
+// gave 6.8-7.7e-6 K: the rounding of the FP32 temperatures themselves.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "btpm_internal.h"
+
+namespace btpm_lin {
+
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef float f4 __attribute__((ext_vector_type(4)));
+
+constexpr float kScale = 32768.0f;
+constexpr int kFrags = 12;              // 6 blocks x (hi, lo), 64 lanes x 8 halves each
+constexpr int kFrag = 64 * 8;           // halves per fragment
+// an operator in memory (halves): main[12], tail[12] (the last block's steps),
+// init[2] (base(1..8) of the first block from the nodes), then float g[8]
+constexpr int kTail = kFrags * kFrag;
+constexpr int kInit = 2 * kFrags * kFrag;
+constexpr int kGain = kInit + 2 * kFrag;
+static_assert(kGain + 16 <= BTPM_LIN_OP, "operator size");
+
+// block b of the product: output tile and input chunk
+constexpr int kBlkTile[6] = {0, 1, 1, 2, 2, 3};
+constexpr int kBlkChunk[6] = {0, 0, 1, 0, 1, 1};
+
+// node held by slot q of group g (0: a surface slot)
+__device__ __forceinline__ int slot_node(int g, int q) {
+  return q < 2 ? 0 : q < 4 ? 1 + 2 * g + (q - 2) : 9 + 16 * (q / 4 - 1) + 4 * g + (q & 3);
+}
+
+// fp16 hi / lo halves of 2^-15 x
+__device__ __forceinline__ void split2(float x, _Float16& hi, _Float16& lo) {
+  hi = (_Float16)fmaf(x, 1.0f / kScale, 0.0f);
+  lo = (_Float16)fmaf(x, 1.0f / kScale, -(float)hi);
+}
+
+// u <- operator u for NT tiles of 16 columns; frag(i) gives fragment i (block
+// i/2, hi then lo) of the lane
+template <int NT, class Frag>
+__device__ __forceinline__ void linear_block(float (&u)[NT][16], Frag frag) {
+  h8 bh[NT][2], bl[NT][2];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        _Float16 a, b;
+        split2(u[t][8 * h + j], a, b);
+        bh[t][h][j] = a;
+        bl[t][h][j] = b;
+      }
+#pragma unroll
+  for (int ot = 0; ot < 4; ++ot) {
+    f4 acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    h8 ahi[2], alo[2];
+#pragma unroll
+    for (int b = 0; b < 6; ++b)
+      if (kBlkTile[b] == ot) {
+        ahi[kBlkChunk[b]] = frag(2 * b);
+        alo[kBlkChunk[b]] = frag(2 * b + 1);
+      }
+    // small products first
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+#pragma unroll
+      for (int b = 0; b < 6; ++b)
+        if (kBlkTile[b] == ot)
+#pragma unroll
+          for (int t = 0; t < NT; ++t) {
+            const int h = kBlkChunk[b];
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(p == 0 ? alo[h] : ahi[h],
+                                                            p == 1 ? bl[t][h] : bh[t][h], acc[t],
+                                                            0, 0, 0);
+          }
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) u[t][4 * ot + i] = acc[t][i];
+  }
+}
+
+// base(1..8) of a rotation's first block from the nodes (surface slots zero)
+template <int NT>
+__device__ __forceinline__ void linear_init(float (&u)[NT][16], h8 ahi, h8 alo) {
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    h8 bh, bl;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      _Float16 a, b;
+      split2(u[t][j], a, b);
+      bh[j] = a;
+      bl[j] = b;
+    }
+    f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bh, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bl, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bh, acc, 0, 0, 0);
+    u[t][0] = acc[0];
+    u[t][1] = acc[1];
+  }
+}
+
+__device__ __forceinline__ void swap32(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false,
+                                                  false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap16(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false,
+                                                  false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+// transposes (register i, lane group g) of four registers; its own inverse
+__device__ __forceinline__ void transpose4(float& x0, float& x1, float& x2, float& x3) {
+  swap32(x0, x2);
+  swap32(x1, x3);
+  swap16(x0, x1);
+  swap16(x2, x3);
+}
+
+// Surface slots <-> one column per lane.  64 columns (NT = 4): lane 16 t + c
+// takes the 8 surface values of column c of tile t.  16 columns (NT = 1):
+// every lane group takes all 8 values of its column.
+__device__ __forceinline__ void surface_out(const float (&u)[4][16], float (&w)[8]) {
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    float x0 = u[0][q], x1 = u[1][q], x2 = u[2][q], x3 = u[3][q];
+    transpose4(x0, x1, x2, x3);
+    w[q] = x0;
+    w[2 + q] = x1;
+    w[4 + q] = x2;
+    w[6 + q] = x3;
+  }
+}
+__device__ __forceinline__ void surface_in(float (&u)[4][16], const float (&w)[8]) {
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    float x0 = w[q], x1 = w[2 + q], x2 = w[4 + q], x3 = w[6 + q];
+    transpose4(x0, x1, x2, x3);
+    u[0][q] = x0;
+    u[1][q] = x1;
+    u[2][q] = x2;
+    u[3][q] = x3;
+  }
+}
+__device__ __forceinline__ void surface_out(const float (&u)[1][16], float (&w)[8]) {
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    float a = u[0][q], b = a;
+    swap32(a, b);  // a: groups 0, 1 twice; b: groups 2, 3 twice
+    float a2 = a, b2 = b;
+    swap16(a, a2);
+    swap16(b, b2);
+    w[q] = a;
+    w[2 + q] = a2;
+    w[4 + q] = b;
+    w[6 + q] = b2;
+  }
+}
+__device__ __forceinline__ void surface_in(float (&u)[1][16], const float (&w)[8]) {
+  const int g = (int)(threadIdx.x & 63) >> 4;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const float lo = (g & 1) ? w[2 + q] : w[q];
+    const float hi = (g & 1) ? w[6 + q] : w[4 + q];
+    u[0][q] = (g & 2) ? hi : lo;
+  }
+}
+
+// One tile's nodes from / to profile records (57 nodes, offsets from tref)
+typedef float uf4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef float uf2 __attribute__((ext_vector_type(2), aligned(4)));
+typedef __attribute__((address_space(1))) float gf;
+
+__device__ __forceinline__ void load_nodes(const gf* rec, int g, float tref, float (&u)[16]) {
+  const uf2 a = *reinterpret_cast<const __attribute__((address_space(1))) uf2*>(rec + 1 + 2 * g);
+  u[0] = u[1] = 0.0f;
+  u[2] = (a.x - tref) * kScale;
+  u[3] = (a.y - tref) * kScale;
+#pragma unroll
+  for (int t = 1; t < 4; ++t) {
+    const uf4 v = *reinterpret_cast<const __attribute__((address_space(1))) uf4*>(
+        rec + 9 + 16 * (t - 1) + 4 * g);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) u[4 * t + i] = (v[i] - tref) * kScale;
+  }
+}
+// (node 56 is written as the copy of node 55, the zero-flux bottom)
+__device__ __forceinline__ void store_nodes(gf* rec, int g, float tref, const float (&u)[16]) {
+  auto node = [&](float x) { return fmaf(x, 1.0f / kScale, tref); };
+  *reinterpret_cast<__attribute__((address_space(1))) uf2*>(rec + 1 + 2 * g) =
+      uf2{node(u[2]), node(u[3])};
+#pragma unroll
+  for (int t = 1; t < 4; ++t) {
+    uf4 v = {node(u[4 * t]), node(u[4 * t + 1]), node(u[4 * t + 2]), node(u[4 * t + 3])};
+    if (t == 3 && g == 3) v[3] = v[2];
+    *reinterpret_cast<__attribute__((address_space(1))) uf4*>(rec + 9 + 16 * (t - 1) + 4 * g) = v;
+  }
+}
+
+}  // namespace btpm_lin

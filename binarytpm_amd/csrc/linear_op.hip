@@ -1,0 +1,118 @@
+// linear_op.hip -- host side of linear_block.h: the matrices of eight explicit
+// conduction steps for one FTCS number, split and packed as the fragments the
+// matrix instructions read.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+
+#include "linear_block.h"
+#include "runtime.h"
+
+namespace btpm {
+namespace {
+constexpr int N = BTPM_NX - 1;       // interior nodes 1..55
+constexpr int B = BTPM_BLK;
+constexpr int L = N + B;             // inputs: nodes, then u0(0..7); outputs: nodes, base(1..8)
+
+// entry of a slot: node - 1, or N + surface index, or -1 (node 56)
+int slot_entry(int g, int q) {
+  if (q < 2) return N + 2 * g + q;
+  const int n = q < 4 ? 1 + 2 * g + (q - 2) : 9 + 16 * (q / 4 - 1) + 4 * g + (q & 3);
+  return n <= N ? n - 1 : -1;
+}
+
+// one FTCS step of the nodes with surface value s (node 0) and the zero-flux
+// bottom u[NX] = u[NX-1]
+void ftcs(double (&u)[N], double r, double s) {
+  double before = s;
+  for (int i = 0; i < N; ++i) {
+    const double cur = u[i], next = i + 1 < N ? u[i + 1] : cur;
+    u[i] = cur + r * (next - 2.0 * cur + before);
+    before = cur;
+  }
+}
+
+// out[row][entry] of `steps` steps: nodes after them and, with `responses`,
+// node 1 after 1..8 further steps without surface input
+void respond(double r, int steps, bool responses, double (&out)[L][L]) {
+  std::memset(out, 0, sizeof out);
+  for (int e = 0; e < L; ++e) {
+    double u[N] = {0.0};
+    if (e < N) u[e] = 1.0;
+    for (int k = 0; k < steps; ++k) ftcs(u, r, e == N + k ? 1.0 : 0.0);
+    for (int i = 0; i < N; ++i) out[i][e] = u[i];
+    if (!responses) continue;
+    for (int s = 0; s < B; ++s) {
+      ftcs(u, r, 0.0);
+      out[N + s][e] = u[0];
+    }
+  }
+}
+
+// hi and lo of every entry times 2^15, the rounding of the low halves carried
+// along the row from its largest entry to its smallest
+void split_rows(const double (&m)[L][L], _Float16 (&hi)[L][L], _Float16 (&lo)[L][L]) {
+  for (int i = 0; i < L; ++i) {
+    int by[L];
+    for (int j = 0; j < L; ++j) by[j] = j;
+    std::sort(by, by + L, [&](int a, int b) { return std::fabs(m[i][a]) > std::fabs(m[i][b]); });
+    double carry = 0.0;
+    for (int k = 0; k < L; ++k) {
+      const int j = by[k];
+      const double x = m[i][j] * btpm_lin::kScale;
+      hi[i][j] = (_Float16)x;
+      if (m[i][j] == 0.0) {
+        lo[i][j] = (_Float16)0.0f;
+        continue;
+      }
+      const double w = x - (double)hi[i][j] + carry;
+      lo[i][j] = (_Float16)w;
+      carry = w - (double)lo[i][j];
+    }
+  }
+}
+
+// the fragment pair (hi, lo) of output tile t and input chunk h
+void pack(const _Float16 (&hi)[L][L], const _Float16 (&lo)[L][L], int t, int h, _Float16* out) {
+  for (int lane = 0; lane < 64; ++lane)
+    for (int j = 0; j < 8; ++j) {
+      const int m = lane & 15;
+      const int row = slot_entry(m >> 2, 4 * t + (m & 3)), col = slot_entry(lane >> 4, 8 * h + j);
+      const bool in = row >= 0 && col >= 0;
+      out[lane * 8 + j] = in ? hi[row][col] : (_Float16)0.0f;
+      out[btpm_lin::kFrag + lane * 8 + j] = in ? lo[row][col] : (_Float16)0.0f;
+    }
+}
+}  // namespace
+
+void linear_operator(float rf, int ntau, _Float16* op) {
+  const double r = (double)rf;
+  static thread_local double m[L][L];
+  static thread_local _Float16 hi[L][L], lo[L][L];
+  std::fill(op, op + BTPM_LIN_OP, (_Float16)0.0f);
+  respond(r, B, true, m);
+  split_rows(m, hi, lo);
+  for (int b = 0; b < 6; ++b) pack(hi, lo, btpm_lin::kBlkTile[b], btpm_lin::kBlkChunk[b], op + 2 * b * btpm_lin::kFrag);
+  // the last block's steps: nodes only
+  respond(r, ntau - (nblocks(ntau) - 1) * B, false, m);
+  split_rows(m, hi, lo);
+  for (int b = 0; b < 6; ++b)
+    pack(hi, lo, btpm_lin::kBlkTile[b], btpm_lin::kBlkChunk[b], op + btpm_lin::kTail + 2 * b * btpm_lin::kFrag);
+  // base(1..8) of the first block from the nodes (no steps before it)
+  respond(r, 0, true, m);
+  for (int i = 0; i < N; ++i)
+    for (int j = 0; j < L; ++j) m[i][j] = 0.0;
+  split_rows(m, hi, lo);
+  pack(hi, lo, 0, 0, op + btpm_lin::kInit);
+  // g(k): node 1, k + 1 steps after a unit surface value
+  float g[B];
+  double u[N] = {0.0};
+  for (int k = 0; k < B; ++k) {
+    ftcs(u, r, k == 0 ? 1.0 : 0.0);
+    g[k] = (float)u[0];
+  }
+  std::memcpy(op + btpm_lin::kGain, g, sizeof g);
+}
+}  // namespace btpm

@@ -541,3 +541,24 @@ def test_full_size_config0_parity(ctx):
     absorbed = 0.9 * case.illum.astype(np.float64).sum(1)
     emitted = (ES * gpu.astype(np.float64) ** 4).sum(1)
     assert (np.abs(absorbed - emitted) / absorbed).max() < 1e-2
+
+
+def test_trial_class_leaves(rough80):
+    """A rotation cap below the tuner's trial length: the smooth class under
+    trial leaves with its last set while the crater set still runs, and the
+    graph is captured for what is left."""
+    case, crater = rough80
+    p = th.params(650, case.rot_period, tacc=0.01, max_rev=4)
+    cm = th.CraterModel(vf=crater["vf"], shadow=crater["shadow"], cosang=crater["cosang"],
+                        solar=crater["solar"], multiple=True, scatter_acc=1e-4)
+    with th.Context(0) as c2:  # a fresh context: nothing tuned yet
+        shape = th.Shape(c2, p, case.illum, 0.1, crater=cm)
+        out = []
+        for tune in (True, False):
+            s = th.Solve(c2, shape, 200.0, with_craters=True)
+            th.batch_run(c2, [s], th.batch_opts(autotune=tune, rotations_per_sync=1))
+            assert s.info().rotations == 4 and s.info().crater_rotations == 4
+            out.append(s.crater_temps())
+            s.close()
+        assert np.array_equal(out[0], out[1])
+        shape.close()

@@ -45,4 +45,21 @@ __device__ __forceinline__ double sbc_newton(double src, double m1, double t1, d
   return newton_finish(K, m1, es, x, d0, tol, cap);
 }
 
+// The first iteration split so that what depends on node 1 (the last value
+// to become known) is one FMA: with x0 the start, rk = 1 / g'(x0) and
+//   a = x0 + (src - m1 x0 - es x0^4) rk,   b = m1 rk
+// the first iterate is a + b t1.  a and b are ready before the step's node 1.
+struct FirstIterate {
+  double x0, a, b;
+};
+__device__ __forceinline__ FirstIterate newton_first(double x0, double src, double m1, double es) {
+  FirstIterate f;
+  f.x0 = fmax(x0, 1.0);
+  const double ex3 = es * ((f.x0 * f.x0) * f.x0);
+  const double rk = __builtin_amdgcn_rcp(fma(4.0, ex3, m1));
+  f.a = fma(fma(-ex3, f.x0, fma(-m1, f.x0, src)), rk, f.x0);
+  f.b = m1 * rk;
+  return f;
+}
+
 }  // namespace btpm_dev

@@ -52,6 +52,12 @@
 // ((1 - 2r)^-8 * 1e4 K < 3e38 needs 1 - 2r > 5.6e-5)
 #define BTPM_R_MAX 0.49995
 
+// halves of one 8-step conduction operator (linear_block.h): 12 + 12 + 2
+// matrix fragments of 512 halves and 8 floats, padded to 256 bytes
+#define BTPM_LIN_OP (26 * 512 + 128)
+// fewest columns per tile of the operator's smooth conduction kernels
+#define BTPM_LIN_MIN 16
+
 // kind of a column set
 enum { BTPM_SET_SMOOTH = 0, BTPM_SET_CRATER = 1 };
 
@@ -84,6 +90,7 @@ struct btpm_set_dev {
   float* qext;        // [nb][ncols][BLK] total flux incl. facet self-heating (or null)
   float* emis;        // [ncols][nb*BLK] esia T^4 for the next rotation (or null),
                       // facet-major for the self-heating SpMM's coalesced reads
+  const void* op;     // 8-step conduction operator of the set's FTCS number (linear_block.h)
   const float* vfA;   // crater: fp16 hi/lo view-factor tiles (see crater kernel)
   // status, written by the kernels
   int* tile_active;   // [ntiles] active groups after this rotation's test

@@ -21,8 +21,27 @@ extern template __global__ void btpm_conduct_smooth<128>(const btpm_tile*, const
                                                          const btpm_status_dev*);
 extern template __global__ void btpm_conduct_smooth<64>(const btpm_tile*, const btpm_set_dev*,
                                                         const btpm_status_dev*);
+// the same on the 8-step operator, 16 NT columns per one-wave workgroup
+// (the register budget of an instantiation comes from this declaration)
+template <int NT>
+__global__ __launch_bounds__(64, 2) void btpm_conduct_smooth_lin(const btpm_tile* tiles, const btpm_set_dev* sets,
+                                        const btpm_status_dev* status);
+extern template __global__ void btpm_conduct_smooth_lin<1>(const btpm_tile*, const btpm_set_dev*,
+                                                           const btpm_status_dev*);
+extern template __global__ void btpm_conduct_smooth_lin<2>(const btpm_tile*, const btpm_set_dev*,
+                                                           const btpm_status_dev*);
+extern template __global__ void btpm_conduct_smooth_lin<4>(const btpm_tile*, const btpm_set_dev*,
+                                                           const btpm_status_dev*);
 extern "C" __global__ void btpm_conduct_crater(const btpm_tile* tiles, const btpm_set_dev* sets,
                                                const btpm_status_dev* status);
+// the same on the 8-step operator, P craters per workgroup
+template <int P>
+__global__ __launch_bounds__((P * BTPM_NS + 63) / 64 * 64) void btpm_conduct_crater_lin(
+    const btpm_tile* tiles, const btpm_set_dev* sets, const btpm_status_dev* status);
+extern template __global__ void btpm_conduct_crater_lin<5>(const btpm_tile*, const btpm_set_dev*,
+                                                           const btpm_status_dev*);
+extern template __global__ void btpm_conduct_crater_lin<2>(const btpm_tile*, const btpm_set_dev*,
+                                                           const btpm_status_dev*);
 extern "C" __global__ void btpm_contract_kernel(const _Float16* vfA, const float* e, float* q,
                                                 int ncol, float unscale_v,
                                                 const float* unscale_p);

@@ -29,6 +29,7 @@
 #include "btpm_internal.h"
 #include "btpm_kernels.h"
 #include "btpm_device.h"
+#include "linear_block.h"
 
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
@@ -368,6 +369,175 @@ template __global__ void btpm_conduct_smooth<64>(const btpm_tile*, const btpm_se
                                                  const btpm_status_dev*);
 
 // ---------------------------------------------------------------------------
+// Smooth facets with one FTCS number for the whole set, on the matrix cores
+// (linear_block.h): one wave per workgroup, 16 NT columns.  NT = 1, 2: four
+// or two lanes solve the surface balances of the same column (the balance is a
+// chain of dependent FP64 operations, so the copies cost no time where a SIMD
+// holds one or two waves, and the set spreads over that many more SIMDs);
+// NT = 4: one column per lane.  A column's arithmetic is the same for each.
+// The operator's 12 fragments stay in registers for the whole rotation.
+// ---------------------------------------------------------------------------
+template <int NT>
+__global__ __launch_bounds__(64, 2) void btpm_conduct_smooth_lin(
+    const btpm_tile* __restrict__ tiles, const btpm_set_dev* __restrict__ sets,
+    const btpm_status_dev* __restrict__ status) {
+  using namespace btpm_lin;
+  constexpr int NX = BTPM_NX;
+  constexpr int W = 16 * NT;
+  const btpm_tile tl = tiles[blockIdx.x];
+  const btpm_set_dev& S = sets[tl.set];
+  const btpm_status_dev st = status[tl.set];
+  if (st.done || st.rev >= S.max_rev) return;
+  const bool check = st.rev > S.check_after;
+  const int lane = (int)threadIdx.x, g = lane >> 4;
+  const int ncols = S.ncols, norder = st.norder;
+  const int last = norder > 0 ? norder - 1 : 0;
+  const int idx = tl.tile * W + lane % W;
+  const bool valid = idx < norder;
+  const int c = S.order[valid ? idx : last];
+  const bool active = valid && (S.inst || !S.frozen[c]);
+  const bool mine = active && lane < W;  // the lane that stores the column
+  const int nwork = __popcll(__ballot(mine));
+  if (nwork == 0) {
+    if (lane == 0) {
+      S.tile_active[tl.tile] = 0;
+      S.tile_work[tl.tile] = 0;
+    }
+    return;
+  }
+  const double m1 = (double)S.m1[c];
+  const double es = (double)S.es;
+  const double tol = (double)S.newton_tol;
+  const int cap = S.newton_cap;
+  const gfloat* __restrict__ srcp = (const gfloat*)(S.qext != nullptr ? S.qext : S.src);
+  const gfloat* __restrict__ Tin = (const gfloat*)S.T;
+  gfloat* __restrict__ Tout = (gfloat*)S.T;
+  gfloat* __restrict__ Eout = (gfloat*)S.emis;
+  const bool has_e = S.emis != nullptr;
+  const float esia = S.esia;
+  const int nb = S.nb, ntau = S.ntau;
+  const size_t bstride = (size_t)ncols * BTPM_BLK;
+  const size_t coff = (size_t)c * BTPM_BLK;
+
+  float nsrc[BTPM_BLK], nprev[BTPM_BLK];
+  load8(srcp + coff, nsrc);
+  load8(Tin + coff, nprev);
+  Surface sf = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+  auto store_block = [&](int b, const float (&out)[BTPM_BLK]) {
+    if (!mine) return;
+    store8(Tout + (size_t)b * bstride + coff, out);
+    if (has_e) {
+      float e[BTPM_BLK];
+#pragma unroll
+      for (int k = 0; k < BTPM_BLK; ++k) e[k] = esia * (out[k] * out[k]) * (out[k] * out[k]);
+      store8(Eout + (size_t)c * nb * BTPM_BLK + (size_t)b * BTPM_BLK, e);  // facet-major
+    }
+  };
+
+  if (S.inst) {  // instantaneous equilibrium (TI = 0), thermal.cpp:1985-2033
+    for (int b = 0; b < nb; ++b) {
+      load8(srcp + (size_t)b * bstride + coff, nsrc);
+      load8(Tin + (size_t)b * bstride + coff, nprev);
+      const int kend = min(BTPM_BLK, ntau - b * BTPM_BLK);
+      float out[BTPM_BLK];
+#pragma unroll
+      for (int k = 0; k < BTPM_BLK; ++k) {
+        out[k] = nprev[k];
+        if (k < kend) {
+          out[k] = (float)sqrt(sqrt((double)nsrc[k] / es));
+          sf.dm = fmaxf(sf.dm, fabsf(out[k] - nprev[k]));
+        }
+      }
+      store_block(b, out);
+    }
+  } else {
+    const GLOBAL_AS h8* __restrict__ op = (const GLOBAL_AS h8*)S.op + lane;
+    h8 A[kFrags];
+#pragma unroll
+    for (int i = 0; i < kFrags; ++i) A[i] = op[i * 64];
+    float gain[BTPM_BLK];
+#pragma unroll
+    for (int k = 0; k < BTPM_BLK; ++k)
+      gain[k] = reinterpret_cast<const float*>(static_cast<const _Float16*>(S.op) + kGain)[k];
+    const gfloat* prof = (const gfloat*)S.prof;
+    auto tile_col = [&](int t) {
+      const int i = tl.tile * W + 16 * t + (lane & 15);
+      return S.order[i < norder ? i : last];
+    };
+    float u[NT][16];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const gfloat* rec = prof + (size_t)tile_col(t) * BTPM_PSTRIDE;
+      load_nodes(rec, g, rec[NX], u[t]);
+    }
+    const gfloat* rec = prof + (size_t)c * BTPM_PSTRIDE;
+    const float Tref = rec[NX];
+    sf.u0 = (rec[0] - Tref) * kScale;
+    const double Trefd = (double)Tref;
+    linear_init<NT>(u, op[2 * kFrags * 64], op[(2 * kFrags + 1) * 64]);
+    float w[BTPM_BLK];
+    surface_out(u, w);
+
+    auto block = [&](int b, auto full_tag) {
+      constexpr bool FULL = decltype(full_tag)::value;
+      const int kend = FULL ? BTPM_BLK : ntau - b * BTPM_BLK;
+      float src[BTPM_BLK], out[BTPM_BLK];
+#pragma unroll
+      for (int k = 0; k < BTPM_BLK; ++k) {
+        src[k] = nsrc[k];
+        out[k] = nprev[k];
+      }
+      if (FULL) {
+        load8(srcp + (size_t)(b + 1) * bstride + coff, nsrc);
+        load8(Tin + (size_t)(b + 1) * bstride + coff, nprev);
+      }
+      surface_steps<FULL>(sf, w, out, src, gain, m1, es, Trefd, tol, cap, kend, [](int) {});
+      store_block(b, out);
+      surface_in(u, w);
+      if constexpr (FULL) {
+        linear_block<NT>(u, [&](int i) { return A[i]; });
+        surface_out(u, w);
+      } else {
+        linear_block<NT>(u, [&](int i) { return (h8)op[(kFrags + i) * 64]; });
+      }
+    };
+    for (int b = 0; b + 1 < nb; ++b) block(b, std::true_type{});
+    block(nb - 1, std::false_type{});
+
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int ct = tile_col(t);
+      if (tl.tile * W + 16 * t + (lane & 15) >= norder || S.frozen[ct]) continue;
+      gfloat* r = (gfloat*)S.prof + (size_t)ct * BTPM_PSTRIDE;
+      store_nodes(r, g, r[NX], u[t]);
+    }
+    if (mine)
+      ((gfloat*)S.prof)[(size_t)c * BTPM_PSTRIDE] = fmaf(sf.u0, 1.0f / kScale, Tref);
+  }
+
+  bool still = mine;
+  if (mine) {
+    S.dmax[c] = sf.dm;
+    if (check && sf.dm < S.tacc) {
+      still = false;
+      if (!S.inst) S.frozen[c] = 1;
+    }
+  }
+  const int nact = __popcll(__ballot(still));
+  if (lane == 0) {
+    S.tile_active[tl.tile] = nact;
+    S.tile_work[tl.tile] = S.inst ? 0 : nwork;
+  }
+}
+
+template __global__ void btpm_conduct_smooth_lin<1>(const btpm_tile*, const btpm_set_dev*,
+                                                    const btpm_status_dev*);
+template __global__ void btpm_conduct_smooth_lin<2>(const btpm_tile*, const btpm_set_dev*,
+                                                    const btpm_status_dev*);
+template __global__ void btpm_conduct_smooth_lin<4>(const btpm_tile*, const btpm_set_dev*,
+                                                    const btpm_status_dev*);
+
+// ---------------------------------------------------------------------------
 // Crater columns: BTPM_CRATERS_WG craters x 100 sub-facets per workgroup of
 // 1024 lanes (lane -> sub-facet column, 24 idle lanes).  Every 8-step block
 // the workgroup evaluates the crater self-heating of all its craters for the
@@ -383,9 +553,10 @@ template __global__ void btpm_conduct_smooth<64>(const btpm_tile*, const btpm_se
 namespace {
 constexpr int kMP = 112;           // padded M (receiving sub-facet j)
 constexpr int kKP = 112;           // padded K (emitting sub-facet i)
-// LDS row stride in halves: 60 dwords, so the 8 rows of one 16-byte fragment
-// read (8 lanes) start 4 banks apart and cover all 32 banks
-constexpr int kLdsK = 120;
+// LDS row stride in halves: 52 dwords, so the 8 rows of one 16-byte fragment
+// read (8 lanes) start at multiples of 4 banks, all different, and cover all
+// 32 banks; k runs to 99 only (three chunks of 32 and the tail 96..99)
+constexpr int kLdsK = 104;
 constexpr int kNP = BTPM_CRATERS_WG * BTPM_BLK;  // 80 columns of the product
 // Q row stride: 1000 columns + 24 idle lanes + 4 floats of padding, so the
 // 8 step rows start in different LDS banks and the product's float4 stores
@@ -412,26 +583,27 @@ constexpr int kNT = kNP / 16;      // 5 N tiles
 //
 // One K chunk of 32 (v_mfma_f32_16x16x32_f16): lane l supplies
 // A[m = l%16][k = 8(l/16) .. +7] and B[k = 8(l/16) .. +7][n = l%16].
-template <int NNT>
-__device__ __forceinline__ void strip_chunk32(const _Float16 (*lds_a)[kMP * kLdsK],
-                                              const _Float16 (*lds_b)[kNP * kLdsK], int am, int k0,
-                                              int nt0, int r, float4_t (&acc)[NNT]) {
-  const half8_t ahi = *reinterpret_cast<const half8_t*>(&lds_a[0][am * kLdsK + k0]);
-  const half8_t alo = *reinterpret_cast<const half8_t*>(&lds_a[1][am * kLdsK + k0]);
+// The low halves lie AH (of A) and BH (of B) halves behind the high ones.
+template <int NNT, int AH, int BH>
+__device__ __forceinline__ void strip_chunk32(const _Float16* lds_a, const _Float16* lds_b, int am,
+                                              int k0, int nt0, int r, float4_t (&acc)[NNT]) {
+  const half8_t ahi = *reinterpret_cast<const half8_t*>(&lds_a[am * kLdsK + k0]);
+  const half8_t alo = *reinterpret_cast<const half8_t*>(&lds_a[AH + am * kLdsK + k0]);
 #pragma unroll
   for (int t = 0; t < NNT; ++t) {
     const int bn = (nt0 + t) * 16 + r;
-    const half8_t bhi = *reinterpret_cast<const half8_t*>(&lds_b[0][bn * kLdsK + k0]);
-    const half8_t blo = *reinterpret_cast<const half8_t*>(&lds_b[1][bn * kLdsK + k0]);
+    const half8_t bhi = *reinterpret_cast<const half8_t*>(&lds_b[bn * kLdsK + k0]);
+    const half8_t blo = *reinterpret_cast<const half8_t*>(&lds_b[BH + bn * kLdsK + k0]);
     acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bhi, acc[t], 0, 0, 0);
     acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, blo, acc[t], 0, 0, 0);
     acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bhi, acc[t], 0, 0, 0);
   }
 }
 
-template <int NNT>
-__device__ __forceinline__ void product_strip(const _Float16 (*lds_a)[kMP * kLdsK],
-                                              const _Float16 (*lds_b)[kNP * kLdsK],
+// (QC: Q row stride; NV: product columns that exist, the rest of the last tile
+// is padding and not stored)
+template <int NNT, int AH, int BH, int QC, int NV>
+__device__ __forceinline__ void product_strip(const _Float16* lds_a, const _Float16* lds_b,
                                               float* lds_q, int mt, int nt0, int lane,
                                               float unscale) {
   constexpr int kFull = BTPM_NS / 32 * 32;  // 96: sub-facets in full chunks of 32
@@ -444,7 +616,7 @@ __device__ __forceinline__ void product_strip(const _Float16 (*lds_a)[kMP * kLds
   const int am = mt * 16 + r;
 #pragma unroll 1
   for (int kt = 0; kt < kFull / 32; ++kt)
-    strip_chunk32<NNT>(lds_a, lds_b, am, kt * 32 + 8 * g, nt0, r, acc);
+    strip_chunk32<NNT, AH, BH>(lds_a, lds_b, am, kt * 32 + 8 * g, nt0, r, acc);
   // the tail k = 96..99 as one v_mfma_f32_16x16x16f16 chunk (k = 4(l/16)..+3):
   // only lanes 0-15 hold sub-facets, the others contribute zero operands
   // instead of reading the zero padding
@@ -454,13 +626,13 @@ __device__ __forceinline__ void product_strip(const _Float16 (*lds_a)[kMP * kLds
 #pragma unroll
     for (int t = 0; t < NNT; ++t) bhi[t] = blo[t] = zero;
     if (g == 0) {
-      ahi = *reinterpret_cast<const half4_t*>(&lds_a[0][am * kLdsK + kFull]);
-      alo = *reinterpret_cast<const half4_t*>(&lds_a[1][am * kLdsK + kFull]);
+      ahi = *reinterpret_cast<const half4_t*>(&lds_a[am * kLdsK + kFull]);
+      alo = *reinterpret_cast<const half4_t*>(&lds_a[AH + am * kLdsK + kFull]);
 #pragma unroll
       for (int t = 0; t < NNT; ++t) {
         const int bn = (nt0 + t) * 16 + r;
-        bhi[t] = *reinterpret_cast<const half4_t*>(&lds_b[0][bn * kLdsK + kFull]);
-        blo[t] = *reinterpret_cast<const half4_t*>(&lds_b[1][bn * kLdsK + kFull]);
+        bhi[t] = *reinterpret_cast<const half4_t*>(&lds_b[bn * kLdsK + kFull]);
+        blo[t] = *reinterpret_cast<const half4_t*>(&lds_b[BH + bn * kLdsK + kFull]);
       }
     }
 #pragma unroll
@@ -475,7 +647,8 @@ __device__ __forceinline__ void product_strip(const _Float16 (*lds_a)[kMP * kLds
 #pragma unroll
     for (int t = 0; t < NNT; ++t) {
       const int bn = (nt0 + t) * 16 + r;
-      float* q = &lds_q[(bn & (BTPM_BLK - 1)) * kQCols + (bn / BTPM_BLK) * BTPM_NS + m0];
+      if (NV % 16 != 0 && bn >= NV) continue;
+      float* q = &lds_q[(bn & (BTPM_BLK - 1)) * QC + (bn / BTPM_BLK) * BTPM_NS + m0];
       *reinterpret_cast<float4*>(q) = make_float4(acc[t][0] * unscale, acc[t][1] * unscale,
                                                   acc[t][2] * unscale, acc[t][3] * unscale);
     }
@@ -486,25 +659,25 @@ __device__ __forceinline__ void product_strip(const _Float16 (*lds_a)[kMP * kLds
 // 7..13 = m tile (value - 7) with n tiles 3-4, 15 = none
 constexpr unsigned long long kStripOfWave = 0xD9FFC852B741A630ull;
 
-__device__ __forceinline__ void crater_product(const _Float16 (*lds_a)[kMP * kLdsK],
-                                               const _Float16 (*lds_b)[kNP * kLdsK],
+template <int AH, int BH, int QC>
+__device__ __forceinline__ void crater_product(const _Float16* lds_a, const _Float16* lds_b,
                                                float* lds_q, int wave, int lane, float unscale) {
   static_assert(kMT == 7 && kNT == 5 && BTPM_CRATER_THREADS == 1024, "strip table shape");
   const int s = (int)((kStripOfWave >> (4 * wave)) & 15ull);
   if (s < kMT)
-    product_strip<3>(lds_a, lds_b, lds_q, s, 0, lane, unscale);
+    product_strip<3, AH, BH, QC, kNP>(lds_a, lds_b, lds_q, s, 0, lane, unscale);
   else if (s < 2 * kMT)
-    product_strip<2>(lds_a, lds_b, lds_q, s - kMT, 3, lane, unscale);
+    product_strip<2, AH, BH, QC, kNP>(lds_a, lds_b, lds_q, s - kMT, 3, lane, unscale);
 }
 
-// Stage VF^T hi/lo ([2][112][112] fp16 in global memory) into LDS.
+// Stage VF^T hi/lo ([2][112][112] fp16 in global memory) into LDS, k < 104.
 __device__ __forceinline__ void stage_vf(const _Float16* src, _Float16 (*lds_a)[kMP * kLdsK],
                                          int tid) {
-  for (int e = tid; e < 2 * kMP * kKP; e += BTPM_CRATER_THREADS) {
-    const int h = e / (kMP * kKP);
-    const int rem = e - h * kMP * kKP;
-    const int m = rem / kKP, k = rem - m * kKP;
-    lds_a[h][m * kLdsK + k] = src[e];
+  for (int e = tid; e < 2 * kMP * kLdsK; e += BTPM_CRATER_THREADS) {
+    const int h = e / (kMP * kLdsK);
+    const int rem = e - h * kMP * kLdsK;
+    const int m = rem / kLdsK, k = rem - m * kLdsK;
+    lds_a[h][rem] = src[(h * kMP + m) * kKP + k];
   }
 }
 }  // namespace
@@ -640,7 +813,7 @@ extern "C" __global__ __launch_bounds__(BTPM_CRATER_THREADS) void btpm_conduct_c
     for (int k = 0; k < BTPM_BLK; ++k) lds_p[k][tid] = nprev[k];
     if (more) load8(Tin + (size_t)(b + 1) * bstride + lane_off(), nprev);
     __syncthreads();
-    crater_product(lds_a, lds_b, lds_q, wave, lane, vf_unscale);
+    crater_product<kMP * kLdsK, kNP * kLdsK, kQCols>(lds_a[0], lds_b[0], lds_q, wave, lane, vf_unscale);
     __syncthreads();
   };
   auto block_tail = [&](int b) {
@@ -759,6 +932,373 @@ extern "C" __global__ __launch_bounds__(BTPM_CRATER_THREADS) void btpm_conduct_c
   }
 }
 
+// ---------------------------------------------------------------------------
+// Crater columns with one FTCS number for the whole set, on the 8-step
+// operator (linear_block.h): P craters x 100 sub-facets per workgroup, lane ->
+// column in the surface steps, four 16-column tiles per wave in the operator's
+// product.  The crater product of block b + 1 needs only the previous
+// rotation's temperatures, so it runs beside the surface steps of block b, a
+// piece of it in each step (its matrix instructions issue into the waits of
+// the balance's dependent FP64 chain), and the emission of block b + 2 is
+// split after them: E and Q are double buffered and a block has one barrier.
+// The fragments that do not change (the wave's m tiles of VF^T, at P = 2
+// the operator too) stay in registers for the whole rotation.P = 5
+// puts 98 % of its lanes to work, two waves to a SIMD; P = 2 spreads few
+// craters over more CUs, one wave to a SIMD.  A 650-step rotation of 80
+// craters takes 232 us at P = 2, 345 us at P = 5 (one crater a workgroup: 259
+// us, four m tiles per wave), where ten craters a workgroup with the steps on
+// the vector ALUs took 663 us; 512 craters 290 / 399 us, 640 craters 534 /
+// 415 us, 5120 craters 1.69 / 1.17 ms (1.19 ms on the vector ALUs).
+// ---------------------------------------------------------------------------
+namespace {
+template <int P>
+struct CraterGroup {
+  static constexpr int kThreads = (P * BTPM_NS + 63) / 64 * 64;
+  static constexpr int kWaves = kThreads / 64;
+  static constexpr int kNT = (P * BTPM_BLK + 15) / 16;  // n tiles of the product
+  static constexpr int kQC = kThreads + 4;              // Q row stride in floats
+  // E rows: the product's columns, and 8 that the idle lanes write
+  static constexpr int kRows = 16 * kNT > 8 * P + 8 ? 16 * kNT : 8 * P + 8;
+  static constexpr int kBH = kRows * kLdsK;             // low halves behind the high
+  static constexpr int kM = (kMT + kWaves - 1) / kWaves;  // m tiles per wave
+  // two waves share a SIMD at P = 5 (256 registers each): the operator's
+  // fragments are read from LDS there
+  static constexpr bool kOpLds = P > 2;
+};
+
+// A fragments of one m tile of VF^T: three K chunks of 32 and the tail 96..99
+// as a fourth whose other slots are zero.  (A 16x16x16 product for the tail
+// right behind the 16x16x32 ones it adds to gave wrong rows 4g, 4g + 1: the
+// two have different pass counts, so they are not chained here.)
+struct VfFrag {
+  half8_t hi[4], lo[4];
+};
+__device__ __forceinline__ VfFrag load_vf(const _Float16* vfA, int mt, int lane) {
+  const int r = lane & 15, g = lane >> 4;
+  const _Float16* row = vfA + (size_t)(mt * 16 + r) * kKP;
+  VfFrag f;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    f.hi[c] = *reinterpret_cast<const half8_t*>(row + 32 * c + 8 * g);
+    f.lo[c] = *reinterpret_cast<const half8_t*>(row + kMP * kKP + 32 * c + 8 * g);
+  }
+  const half8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};  // k >= 100 is zero in the tiles
+  f.hi[3] = g == 0 ? *reinterpret_cast<const half8_t*>(row + 96) : zero;
+  f.lo[3] = g == 0 ? *reinterpret_cast<const half8_t*>(row + kMP * kKP + 96) : zero;
+  return f;
+}
+
+// One piece of the product is K chunk c of n tile t for the wave's M m tiles
+// (mt0, mt0 + step, ...).  Nothing in it branches, so a piece can be scheduled
+// among other work: lanes whose Q does not exist store it behind the row, and
+// in the tail chunk the lanes of g > 0 read entries that meet zeros in A (of
+// the same column, so a NaN there is one already).
+struct EFrag {
+  half8_t hi, lo;
+};
+template <int P>
+__device__ __forceinline__ EFrag load_e(const _Float16* lds_b, int t, int c, int lane) {
+  using G = CraterGroup<P>;
+  const int r = lane & 15, g = lane >> 4;
+  const _Float16* row = lds_b + (16 * t + r) * kLdsK + (c < 3 ? 32 * c + 8 * g : 96);
+  return EFrag{*reinterpret_cast<const half8_t*>(row),
+               *reinterpret_cast<const half8_t*>(row + G::kBH)};
+}
+template <int P, int M>
+__device__ __forceinline__ void product_piece(const VfFrag (&a)[M], const EFrag& e,
+                                              float4_t (&acc)[M], int t, int c, int mt0, int step,
+                                              float* lds_q, int lane, float unscale) {
+  using G = CraterGroup<P>;
+  const int r = lane & 15, g = lane >> 4;
+  if (c == 0)
+#pragma unroll
+    for (int m = 0; m < M; ++m) acc[m] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int p = 0; p < 3; ++p)
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+      acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(p == 0 ? a[m].lo[c] : a[m].hi[c],
+                                                      p == 1 ? e.lo : e.hi, acc[m], 0, 0, 0);
+  if (c < 3) return;
+  const int bn = 16 * t + r;  // product column: crater bn / 8, step bn % 8
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    const int mt = mt0 + m * step, m0 = mt * 16 + 4 * g;
+    const int col = m0 < BTPM_NS && bn < P * BTPM_BLK ? (bn / BTPM_BLK) * BTPM_NS + m0 : G::kThreads;
+    *reinterpret_cast<float4*>(&lds_q[(bn & (BTPM_BLK - 1)) * G::kQC + col]) =
+        make_float4(acc[m][0] * unscale, acc[m][1] * unscale, acc[m][2] * unscale,
+                    acc[m][3] * unscale);
+  }
+}
+}  // namespace
+
+template <int P>
+__global__ __launch_bounds__((P * BTPM_NS + 63) / 64 * 64) void btpm_conduct_crater_lin(
+    const btpm_tile* __restrict__ tiles, const btpm_set_dev* __restrict__ sets,
+    const btpm_status_dev* __restrict__ status) {
+  using namespace btpm_lin;
+  using G = CraterGroup<P>;
+  constexpr int NX = BTPM_NX, NS = BTPM_NS, TH = G::kThreads;
+  __shared__ __align__(16) _Float16 lds_b[2][2 * G::kBH];
+  __shared__ __align__(16) float lds_q[2][BTPM_BLK * G::kQC];
+  __shared__ float lds_t[2][BTPM_BLK][TH];  // T_prev of the next two blocks
+  __shared__ __align__(16) _Float16 lds_op[G::kOpLds ? kFrags * kFrag : 8];
+  __shared__ unsigned lds_cmax[P];
+  __shared__ int lds_cnt;
+
+  const btpm_tile tl = tiles[blockIdx.x];
+  const btpm_set_dev& S = sets[tl.set];
+  const btpm_status_dev st = status[tl.set];
+  if (st.done || st.rev >= S.max_rev) return;
+  const bool check = st.rev > S.check_after;
+  const int tid = (int)threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g4 = lane >> 4;
+  const int norder = st.norder;
+  const int last = norder > 0 ? norder - 1 : 0;
+  // local column -> column through the compacted order; idle lanes and slots
+  // past its end mirror a valid crater's column
+  auto column = [&](int lcol) {
+    const int l = lcol < P * NS ? lcol : P * NS - 1;
+    const int slot = tl.tile * P + l / NS;
+    return S.order[slot < norder ? slot : last] * NS + l % NS;
+  };
+  const int lc = tid < P * NS ? tid : P * NS - 1;
+  const int lcr = lc / NS, j = lc - lcr * NS;
+  const int c = column(tid);
+  const int gr = c / NS;
+  const bool active = tid < P * NS && tl.tile * P + lcr < norder && !S.frozen[gr];
+  const int nwork = __syncthreads_count(active);
+  if (nwork == 0) {
+    if (tid == 0) {
+      S.tile_active[tl.tile] = 0;
+      S.tile_work[tl.tile] = 0;
+    }
+    return;
+  }
+  if (tid < P) lds_cmax[tid] = 0u;
+  // E rows of the last n tile's padding and Q slots of the idle lanes are
+  // never written by a block
+  for (int e = tid; e < 4 * G::kBH; e += TH) (&lds_b[0][0])[e] = (_Float16)0.0f;
+  if (tid >= P * NS)
+    for (int k = 0; k < BTPM_BLK; ++k) lds_q[0][k * G::kQC + tid] = lds_q[1][k * G::kQC + tid] = 0.0f;
+  if constexpr (G::kOpLds)
+    for (int e = tid; e < kFrags * 64; e += TH)
+      reinterpret_cast<h8*>(lds_op)[e] = static_cast<const h8*>(S.op)[e];
+  VfFrag vf[G::kM];
+#pragma unroll
+  for (int m = 0; m < G::kM; ++m)  // past the last m tile: any tile, its rows are not stored
+    vf[m] = load_vf(reinterpret_cast<const _Float16*>(S.vfA), min(wave + m * G::kWaves, kMT - 1),
+                    lane);
+  const double m1 = (double)S.m1[gr];
+  const double es = (double)S.es, tol = (double)S.newton_tol;
+  const int cap = S.newton_cap;
+  const float esia = S.esia;
+  const float vf_unscale = S.vf_unscale;
+  const int nb = S.nb, ntau = S.ntau;
+  const size_t bstride = (size_t)S.ncols * BTPM_BLK;
+  const gfloat* srcp = (const gfloat*)S.src + (size_t)c * BTPM_BLK;
+  const gfloat* Tin = (const gfloat*)S.T + (size_t)c * BTPM_BLK;
+  gfloat* Tout = (gfloat*)S.T + (size_t)c * BTPM_BLK;
+  Surface sf = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+  __syncthreads();  // the cleared E rows, the operator
+
+  // emission of a block, fp16 hi / lo, into E buffer i (idle lanes: rows 8P..)
+  _Float16* const eb = &lds_b[0][(tid / NS * BTPM_BLK) * kLdsK + tid % NS];
+  auto split_e = [&](int i, const float (&t)[BTPM_BLK]) {
+#pragma unroll
+    for (int k = 0; k < BTPM_BLK; ++k) {
+      const float e = esia * (t[k] * t[k]) * (t[k] * t[k]);
+      const _Float16 hi = (_Float16)e;
+      _Float16* p = eb + i * 2 * G::kBH + k * kLdsK;
+      p[0] = hi;
+      p[G::kBH] = (_Float16)(e - (float)hi);
+    }
+  };
+  constexpr int kPieces = 4 * G::kNT;          // of the product, spread over the 8 steps
+  constexpr int kPer = (kPieces + 7) / 8;      // at most in one step
+  auto first_piece = [](int k) { return kPieces * k / 8; };
+  float4_t acc[G::kM];
+  EFrag ef[kPer];
+  // the E fragments of step k's pieces, read a step ahead; the pieces themselves
+  auto load_pieces = [&](int i, int k) {
+#pragma unroll
+    for (int q = 0; q < kPer; ++q)
+      if (first_piece(k) + q < first_piece(k + 1))
+        ef[q] = load_e<P>(lds_b[i], (first_piece(k) + q) / 4, (first_piece(k) + q) % 4, lane);
+  };
+  auto run_pieces = [&](int i, int k) {
+#pragma unroll
+    for (int q = 0; q < kPer; ++q)
+      if (first_piece(k) + q < first_piece(k + 1))
+        product_piece<P>(vf, ef[q], acc, (first_piece(k) + q) / 4, (first_piece(k) + q) % 4, wave,
+                         G::kWaves, lds_q[i], lane, vf_unscale);
+  };
+  auto product = [&](int i) {
+#pragma unroll
+    for (int k = 0; k < BTPM_BLK; ++k) {
+      load_pieces(i, k);
+      run_pieces(i, k);
+    }
+  };
+
+  if (S.inst) {  // roughness_inst_equilibrium, thermal_GPU.cu:581-641
+    for (int b = 0; b < nb; ++b) {
+      float src[BTPM_BLK], t[BTPM_BLK];
+      load8(srcp + (size_t)b * bstride, src);
+      load8(Tin + (size_t)b * bstride, t);
+      split_e(0, t);
+      __syncthreads();
+      product(0);
+      __syncthreads();
+      const int kend = min(BTPM_BLK, ntau - b * BTPM_BLK);
+#pragma unroll
+      for (int k = 0; k < BTPM_BLK; ++k)
+        if (k < kend) {
+          const float x = (float)sqrt(sqrt((double)(src[k] + lds_q[0][k * G::kQC + tid]) / es));
+          sf.dm = fmaxf(sf.dm, fabsf(x - t[k]));
+          t[k] = x;
+        }
+      if (active) store8(Tout + (size_t)b * bstride, t);
+    }
+  } else {
+    const GLOBAL_AS h8* op = (const GLOBAL_AS h8*)S.op + lane;
+    const h8* lop = reinterpret_cast<const h8*>(lds_op) + lane;
+    h8 A[G::kOpLds ? 1 : kFrags];
+    if constexpr (!G::kOpLds)
+#pragma unroll
+      for (int i = 0; i < kFrags; ++i) A[i] = op[i * 64];
+    float gain[BTPM_BLK];
+#pragma unroll
+    for (int k = 0; k < BTPM_BLK; ++k)
+      gain[k] = reinterpret_cast<const float*>(static_cast<const _Float16*>(S.op) + kGain)[k];
+    const gfloat* prof = (const gfloat*)S.prof;
+    float u[4][16];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const gfloat* rec = prof + (size_t)column(64 * wave + 16 * t + (lane & 15)) * BTPM_PSTRIDE;
+      load_nodes(rec, g4, rec[NX], u[t]);
+    }
+    const gfloat* rec = prof + (size_t)c * BTPM_PSTRIDE;
+    const float Tref = rec[NX];
+    sf.u0 = (rec[0] - Tref) * kScale;
+    linear_init<4>(u, op[2 * kFrags * 64], op[(2 * kFrags + 1) * 64]);
+    float w[BTPM_BLK];
+    surface_out(u, w);
+
+    // T_prev and src of a block (past the last: the last again, never used)
+    auto fetch = [&](const gfloat* p, int b, float (&v)[BTPM_BLK]) {
+      load8(p + (size_t)min(b, nb - 1) * bstride, v);
+    };
+    auto park = [&](int i, const float (&v)[BTPM_BLK]) {
+#pragma unroll
+      for (int k = 0; k < BTPM_BLK; ++k) lds_t[i][k][tid] = v[k];
+      asm volatile("" ::: "memory");  // keep them in LDS, not in VGPRs
+    };
+    float nsrc[BTPM_BLK], nprev[BTPM_BLK];
+    fetch(Tin, 0, nprev);
+    park(0, nprev);
+    split_e(0, nprev);
+    fetch(Tin, 1, nprev);
+    fetch(srcp, 0, nsrc);
+    __syncthreads();
+    product(0);
+    park(1, nprev);
+    split_e(1, nprev);
+    fetch(Tin, 2, nprev);
+    __syncthreads();
+
+    auto block = [&](int b, auto full_tag) {
+      constexpr bool FULL = decltype(full_tag)::value;
+      const int i = b & 1;
+      float tot[BTPM_BLK], t[BTPM_BLK];
+#pragma unroll
+      for (int k = 0; k < BTPM_BLK; ++k) {
+        tot[k] = nsrc[k] + lds_q[i][k * G::kQC + tid];
+        t[k] = lds_t[i][k][tid];
+      }
+      if (FULL) {
+        fetch(srcp, b + 1, nsrc);
+        load_pieces(i ^ 1, 0);
+      }
+      surface_steps<FULL>(sf, w, t, tot, gain, m1, es, (double)Tref, tol, cap,
+                          ntau - b * BTPM_BLK, [&](int k) {
+                            if (!FULL) return;
+                            run_pieces(i ^ 1, k);
+                            if (k + 1 < BTPM_BLK) load_pieces(i ^ 1, k + 1);
+                            // one matrix instruction, then the balance's
+#pragma unroll
+                            for (int q = 0; q < 3 * G::kM * kPer; ++q) {
+                              __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                              __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+                            }
+                          });
+      if (active) store8(Tout + (size_t)b * bstride, t);
+      if (FULL) {
+        park(i, nprev);
+        split_e(i, nprev);
+        fetch(Tin, b + 3, nprev);
+      }
+      surface_in(u, w);
+    };
+    for (int b = 0; b + 1 < nb; ++b) {
+      block(b, std::true_type{});
+      if constexpr (G::kOpLds) {
+        // two tiles at a time: a fragment read from LDS serves both
+        auto frag = [&](int i) { return lop[i * 64]; };
+        linear_block<2>(*reinterpret_cast<float (*)[2][16]>(&u[0]), frag);
+        asm volatile("" ::: "memory");
+        linear_block<2>(*reinterpret_cast<float (*)[2][16]>(&u[2]), frag);
+      } else {
+        linear_block<4>(u, [&](int i) { return A[i]; });
+      }
+      surface_out(u, w);
+      __syncthreads();
+    }
+    block(nb - 1, std::false_type{});
+    {
+      auto frag = [&](int i) { return (h8)op[(kFrags + i) * 64]; };
+      linear_block<2>(*reinterpret_cast<float (*)[2][16]>(&u[0]), frag);
+      asm volatile("" ::: "memory");
+      linear_block<2>(*reinterpret_cast<float (*)[2][16]>(&u[2]), frag);
+    }
+
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int l = 64 * wave + 16 * t + (lane & 15);
+      const int ct = column(l);
+      if (l >= P * NS || tl.tile * P + l / NS >= norder || S.frozen[ct / NS]) continue;
+      gfloat* r = (gfloat*)S.prof + (size_t)ct * BTPM_PSTRIDE;
+      store_nodes(r, g4, r[NX], u[t]);
+    }
+    if (active) ((gfloat*)S.prof)[(size_t)c * BTPM_PSTRIDE] = fmaf(sf.u0, 1.0f / kScale, Tref);
+  }
+
+  // per-crater freeze test (converged kernel, T175706/thermal_GPU.cu:648-692)
+  if (active) atomicMax(&lds_cmax[lcr], __float_as_uint(sf.dm));
+  if (tid == 0) lds_cnt = 0;
+  __syncthreads();
+  if (active && j == 0) {
+    const float cm = __uint_as_float(lds_cmax[lcr]);
+    S.dmax[gr] = cm;
+    bool still = true;
+    if (check && cm < S.tacc) {
+      S.frozen[gr] = 1;
+      still = false;
+    }
+    if (still) atomicAdd(&lds_cnt, 1);
+  }
+  __syncthreads();
+  if (tid == 0) {
+    S.tile_active[tl.tile] = lds_cnt;
+    S.tile_work[tl.tile] = S.inst ? 0 : nwork;
+  }
+}
+
+template __global__ void btpm_conduct_crater_lin<5>(const btpm_tile*, const btpm_set_dev*,
+                                                    const btpm_status_dev*);
+template __global__ void btpm_conduct_crater_lin<2>(const btpm_tile*, const btpm_set_dev*,
+                                                    const btpm_status_dev*);
+
 // Standalone crater self-heating product (tests, tools and the
 // allocation-free entry point):
 //   q[n][j] = sum_i VF(j->i) e[n][i],  n < ncol, with the kernel's own split.
@@ -783,7 +1323,8 @@ extern "C" __global__ __launch_bounds__(BTPM_CRATER_THREADS) void btpm_contract_
     lds_b[1][x] = (_Float16)(v - (float)hi);
   }
   __syncthreads();
-  crater_product(lds_a, lds_b, lds_q, tid >> 6, tid & 63, unscale);
+  crater_product<kMP * kLdsK, kNP * kLdsK, kQCols>(lds_a[0], lds_b[0], lds_q, tid >> 6, tid & 63,
+                                                   unscale);
   __syncthreads();
   for (int x = tid; x < kNP * BTPM_NS; x += BTPM_CRATER_THREADS) {
     const int n = x / BTPM_NS, jj = x - n * BTPM_NS;

@@ -300,6 +300,7 @@ struct btpm_shape {
   // creation, then each solve's RGH; every use is on the context's stream)
   DBuf wfm;
   float vf_unscale = 1.0f;
+  DBuf op;  // 8-step conduction operator when every facet has one FTCS number
   std::vector<float> h_albedo, h_numrevs;
 };
 
@@ -363,6 +364,12 @@ void fill_set_common(btpm_set_dev& d, const btpm_params& p) {
   d.newton_cap = p.newton_cap;
 }
 
+// FTCS number r = dtau/dz^2 of a facet that turns numrevs times a cycle
+float ftcs_number(double numrevs, int ntau) {
+  const double dz = 8.0 / BTPM_NX;
+  return (float)((2.0 * kPi * numrevs / ntau) / (dz * dz));
+}
+
 // per-group coefficients r = dtau/dz^2 and m1 = Gamma sqrt(2 pi n / P)/dz
 void coefficients(const btpm_shape* sh, const btpm_solve* s, std::vector<float>& r,
                   std::vector<float>& m1, int* inst) {
@@ -375,7 +382,7 @@ void coefficients(const btpm_shape* sh, const btpm_solve* s, std::vector<float>&
     const double n = sh->h_numrevs[f];
     const double ti = s->ti_facet.empty() ? s->ti : s->ti_facet[f];
     if (ti != 0.0) all_zero = 0;
-    r[f] = (float)((2.0 * kPi * n / sh->p.ntau) / (dz * dz));
+    r[f] = ftcs_number(n, sh->p.ntau);
     m1[f] = (float)(ti * std::sqrt(2.0 * kPi * n / sh->p.rot_period) / dz);
   }
   *inst = all_zero;
@@ -433,8 +440,9 @@ void build_smooth(btpm_solve* s, hipStream_t st) {
     S->qext.alloc(nser * sizeof(float));
     S->emis.alloc(nser * sizeof(float));
   }
-  // tile arrays for the narrowest tuned width (64 columns per workgroup)
-  S->ntiles = (d.ncols + 63) / 64;
+  // tile arrays for the narrowest width
+  d.op = sh->op.p;
+  S->ntiles = d.op ? (d.ncols + BTPM_LIN_MIN - 1) / BTPM_LIN_MIN : (d.ncols + 63) / 64;
   S->tile_active.alloc(S->ntiles * sizeof(int));
   S->tile_work.alloc(S->ntiles * sizeof(int));
   d.src = S->src.as<float>();
@@ -490,7 +498,8 @@ void build_crater(btpm_solve* s, hipStream_t st) {
   S->frozen.alloc(d.ngroups);
   alloc_order(S.get(), d.ngroups, st);
   S->dmax.alloc(d.ngroups * sizeof(float));
-  S->ntiles = (d.ngroups + BTPM_CRATERS_WG - 1) / BTPM_CRATERS_WG;
+  d.op = sh->op.p;
+  S->ntiles = d.op ? (d.ngroups + 1) / 2 : (d.ngroups + BTPM_CRATERS_WG - 1) / BTPM_CRATERS_WG;
   S->tile_active.alloc(S->ntiles * sizeof(int));
   S->tile_work.alloc(S->ntiles * sizeof(int));
   d.src = S->src.as<float>();
@@ -595,16 +604,29 @@ struct Sched {
   hipGraph_t graph = nullptr;
   hipGraphExec_t phase_exec[4] = {nullptr, nullptr, nullptr, nullptr};
   hipGraph_t phase_graph[4] = {nullptr, nullptr, nullptr, nullptr};
-  DBuf d_tiles_c, d_ids;
+  DBuf d_ids;
   // smooth tiles, one launch per workgroup width (the set on trial, if any,
   // in a launch of its own)
-  struct SmoothList {
-    int width;
+  struct TileList {
+    int width;   // + kLinear: a list of the 8-step operator's kernels
     int n;
     bool trial;
     std::unique_ptr<DBuf> tiles;
   };
-  std::vector<SmoothList> smooth_lists;
+  std::vector<TileList> smooth_lists;
+  // crater tiles, one launch per workgroup shape: width = craters per
+  // workgroup (+ kLinear on the 8-step operator)
+  std::vector<TileList> crater_lists;
+  static constexpr int kLinear = 1 << 16;
+  // columns of the resident smooth sets on the 8-step operator
+  long long linear_cols() const {
+    long long cols = 0;
+    for (auto& kv : slots) {
+      const SetHost* S = kv.second.second;
+      if (S->d.kind == BTPM_SET_SMOOTH && S->d.op) cols += S->d.ncols;
+    }
+    return cols;
+  }
   // smooth sets with facet self-heating, grouped by shape: one tiled SpMM
   // launch per group per rotation
   struct HeatGroup {
@@ -643,7 +665,8 @@ struct Sched {
   // ---- autotuner ----------------------------------------------------------
   // Tile choices per size class, measured on the device:
   //   kind 0: smooth conduction columns per workgroup {256, 128, 64}, per
-  //           column-count class (ceil log2 of the set's columns);
+  //           column-count class (ceil log2 of the set's columns); kind 2: of
+  //           the 8-step operator's kernels {16, 32, 64};
   //   kind 1: facet self-heating kernel {time-lane (0), per-chunk CSR or ELL
   //           64, ELL 32, receiver-grouped} as the shape's layouts allow, per
   //           (log2 nnz, log2 facets, step blocks) class.
@@ -674,7 +697,34 @@ struct Sched {
     while ((1LL << c) < v) ++c;
     return c;
   }
-  static TuneKey smooth_key(const SetHost* S) { return {0, log2_class(S->d.ncols)}; }
+  // The operator's kernels (16, 32 or 64 columns per wave) share a launch, and
+  // what a width costs turns on how many waves all their sets make together:
+  // up to kLinCols columns every width leaves SIMDs without a wave, beyond it
+  // the copies of a column's balance compete, so the two are tuned apart.
+  static constexpr long long kLinCols = 32768;
+  TuneKey smooth_key(const SetHost* S) const {
+    const long long c = log2_class(S->d.ncols);
+    return S->d.op ? TuneKey{2, c | (linear_cols() > kLinCols ? 64 : 0)} : TuneKey{0, c};
+  }
+  static std::vector<int> smooth_candidates(const SetHost* S) {
+    return S->d.op ? std::vector<int>{16, 32, 64} : std::vector<int>{256, 128, 64};
+  }
+  // Craters per workgroup of the operator's crater conduction, for all such
+  // sets of a rotation together: 2 while every workgroup has a CU to itself
+  // (512 craters: 290 us a rotation against 399 us with 5), else 5 (640
+  // craters: 415 us against 534 us with 2, which then takes two rounds).
+  static constexpr long long kPairCraters = 512;
+  int crater_width() const {
+    long long n = 0;
+    for (auto& kv : slots) {
+      const SetHost* S = kv.second.second;
+      if (S->d.kind == BTPM_SET_CRATER && S->d.op) n += ctx->h_status[S->slot].norder;
+    }
+    return n <= kPairCraters ? 2 : 5;
+  }
+  int smooth_default(const SetHost* S) const {
+    return S->d.op ? (linear_cols() > kLinCols ? 64 : 16) : BTPM_SMOOTH_WG;
+  }
   static TuneKey heat_key(const btpm_shape* sh) {
     return {1, (log2_class(sh->nnz) << 40) | (log2_class(sh->nf) << 24) | sh->nb};
   }
@@ -744,10 +794,10 @@ struct Sched {
   // with the big sets beside it (sets are independent: results are the same).
   // Off in tuning trials; in profiled runs the fast rotations are launched
   // after each timed rotation, outside its events.
-  std::vector<SmoothList> fsmooth;
+  std::vector<TileList> fsmooth, fcrater;
   std::vector<HeatGroup> fheat;
-  DBuf fd_tiles_c, fd_ids;
-  int fn_tiles_c = 0, fn_ids = 0;
+  DBuf fd_ids;
+  int fn_ids = 0;
   bool fast_active = false;
   btpm_batch_stats stats{};
   // launch timing (opts.profile): events around each conduction launch
@@ -946,6 +996,14 @@ struct Sched {
     return std::min(S->ntiles, (n + S->d.tile_cols - 1) / S->d.tile_cols);
   }
 
+  int push_list(std::vector<TileList>& to, int w, const std::vector<btpm_tile>& v, bool trial) {
+    if (v.empty()) return 0;
+    TileList l{w, (int)v.size(), trial, std::make_unique<DBuf>()};
+    upload(*l.tiles, v.data(), v.size(), ctx->stream);
+    to.push_back(std::move(l));
+    return to.back().n;
+  }
+
   void rebuild_lists() {
     // tuning: classes present without a decision get a trial; a trial whose
     // sets have all left is dropped (it restarts if the class returns)
@@ -960,7 +1018,7 @@ struct Sched {
       for (auto& kv : slots)
         if (kv.second.second->d.kind == BTPM_SET_SMOOTH) {
           present.insert(smooth_key(kv.second.second));
-          want_trial(smooth_key(kv.second.second), {256, 128, 64});
+          want_trial(smooth_key(kv.second.second), smooth_candidates(kv.second.second));
         }
       for (auto& kv : by_shape)
         if (kv.first->force_heat < 0) {
@@ -970,43 +1028,47 @@ struct Sched {
       while (!trials.empty() && !present.count(trials.front().key)) trials.pop_front();
       if (!trials.empty()) trials.front().units = 0.0;
     }
-    std::map<int, std::vector<btpm_tile>> ts;
-    std::vector<btpm_tile> ts_trial, tc;
+    std::map<int, std::vector<btpm_tile>> ts, tc;
+    std::vector<btpm_tile> ts_trial;
     std::vector<int> ids;
+    const int cw = crater_width();
     for (auto& kv : slots) {
       SetHost* S = kv.second.second;
       ids.push_back(S->slot);
       const int unfrozen = ctx->h_status[S->slot].norder;
+      auto set_width = [&](int w) {
+        if (S->d.tile_cols == w) return;  // the status kernel reads the width too
+        S->d.tile_cols = w;
+        HIPCHK(hipMemcpyAsync(ctx->d_sets + S->slot, &S->d, sizeof(btpm_set_dev),
+                              hipMemcpyHostToDevice, ctx->stream));
+      };
       if (S->d.kind == BTPM_SET_SMOOTH) {
         const TuneKey k = smooth_key(S);
-        const int w = choice(k, BTPM_SMOOTH_WG);
-        if (S->d.tile_cols != w) {  // the status kernel reads the width too
-          S->d.tile_cols = w;
-          HIPCHK(hipMemcpyAsync(ctx->d_sets + S->slot, &S->d, sizeof(btpm_set_dev),
-                                hipMemcpyHostToDevice, ctx->stream));
-        }
+        const int w = choice(k, smooth_default(S));
+        set_width(w);
         S->listed = needed_tiles(S);
         const bool tr = on_trial(k);
         if (tr) trials.front().units += unfrozen;
-        for (int t = 0; t < S->listed; ++t) (tr ? ts_trial : ts[w]).push_back(btpm_tile{S->slot, t});
+        for (int t = 0; t < S->listed; ++t) (tr ? ts_trial : ts[S->d.op ? kLinear + w : w]).push_back(btpm_tile{S->slot, t});
       } else {
         // only the tiles the compacted order[] can fill (it only shrinks)
+        if (S->d.op) set_width(cw);
         S->listed = needed_tiles(S);
-        for (int t = 0; t < S->listed; ++t) tc.push_back(btpm_tile{S->slot, t});
+        auto& v = tc[S->d.op ? kLinear + cw : BTPM_CRATERS_WG];
+        for (int t = 0; t < S->listed; ++t) v.push_back(btpm_tile{S->slot, t});
       }
     }
     smooth_lists.clear();
-    n_tiles_s = 0;
+    crater_lists.clear();
+    n_tiles_s = n_tiles_c = 0;
     auto add_list = [&](int w, const std::vector<btpm_tile>& v, bool trial) {
-      if (v.empty()) return;
-      SmoothList l{w, (int)v.size(), trial, std::make_unique<DBuf>()};
-      upload(*l.tiles, v.data(), v.size(), ctx->stream);
-      n_tiles_s += l.n;
-      smooth_lists.push_back(std::move(l));
+      n_tiles_s += push_list(smooth_lists, w, v, trial);
     };
-    if (!ts_trial.empty()) add_list(choice(trials.front().key, BTPM_SMOOTH_WG), ts_trial, true);
+    if (!ts_trial.empty())
+      add_list((trials.front().key.first == 2 ? kLinear : 0) + choice(trials.front().key, 0),
+               ts_trial, true);
     for (auto& kv : ts) add_list(kv.first, kv.second, false);
-    n_tiles_c = (int)tc.size();
+    for (auto& kv : tc) n_tiles_c += push_list(crater_lists, kv.first, kv.second, false);
     n_ids = (int)ids.size();
     heat.clear();
     for (auto& kv : by_shape) {
@@ -1027,39 +1089,35 @@ struct Sched {
       }
       heat.push_back(std::move(g));
     }
-    upload(d_tiles_c, tc.data(), tc.size(), ctx->stream);
     upload(d_ids, ids.data(), ids.size(), ctx->stream);
     rebuild_fast();
   }
 
   void rebuild_fast() {
     fsmooth.clear();
+    fcrater.clear();
     fheat.clear();
-    fn_tiles_c = fn_ids = 0;
+    fn_ids = 0;
     fast_active = false;
     if (opt.fast_extra <= 0 || tuning()) return;
     int max_cols = 0;
     for (auto& kv : slots) max_cols = std::max(max_cols, kv.second.second->d.ncols);
     auto fast = [&](const SetHost* S) { return 8LL * S->d.ncols <= max_cols; };
-    std::map<int, std::vector<btpm_tile>> ts;
-    std::vector<btpm_tile> tc;
+    std::map<int, std::vector<btpm_tile>> ts, tc;
     std::vector<int> ids;
     std::map<btpm_shape*, std::vector<int>> by_shape;
     for (auto& kv : slots) {
       const SetHost* S = kv.second.second;
       if (!fast(S)) continue;
       ids.push_back(S->slot);
-      auto& v = S->d.kind == BTPM_SET_SMOOTH ? ts[S->d.tile_cols] : tc;
+      auto& v = (S->d.kind == BTPM_SET_SMOOTH ? ts : tc)[(S->d.op ? kLinear : 0) + S->d.tile_cols];
       for (int t = 0; t < S->listed; ++t) v.push_back(btpm_tile{S->slot, t});
       if (S->d.kind == BTPM_SET_SMOOTH && S->d.qext)
         by_shape[kv.second.first->shape].push_back(S->slot);
     }
     if (ids.empty()) return;
-    for (auto& kv : ts) {
-      SmoothList l{kv.first, (int)kv.second.size(), false, std::make_unique<DBuf>()};
-      upload(*l.tiles, kv.second.data(), kv.second.size(), ctx->stream);
-      fsmooth.push_back(std::move(l));
-    }
+    for (auto& kv : ts) push_list(fsmooth, kv.first, kv.second, false);
+    for (auto& kv : tc) push_list(fcrater, kv.first, kv.second, false);
     for (auto& kv : by_shape) {
       HeatGroup g{kv.first, (int)kv.second.size(), std::make_unique<DBuf>()};
       upload(*g.slots, kv.second.data(), kv.second.size(), ctx->stream);
@@ -1067,9 +1125,7 @@ struct Sched {
         if (m.shape == kv.first) g.code = m.code;
       fheat.push_back(std::move(g));
     }
-    fn_tiles_c = (int)tc.size();
     fn_ids = (int)ids.size();
-    upload(fd_tiles_c, tc.data(), tc.size(), ctx->stream);
     upload(fd_ids, ids.data(), ids.size(), ctx->stream);
     fast_active = true;
   }
@@ -1119,10 +1175,19 @@ struct Sched {
         if (g.trial) trial_event(st, 1);
       }
     } else if (ph == 1) {
-      for (const SmoothList& l : fast ? fsmooth : smooth_lists) {
+      for (const TileList& l : fast ? fsmooth : smooth_lists) {
         const btpm_tile* t = l.tiles->as<btpm_tile>();
         if (l.trial) trial_event(st, 0);
-        if (l.width == 64)
+        if (l.width == kLinear + 16)
+          hipLaunchKernelGGL(btpm_conduct_smooth_lin<1>, dim3(l.n), dim3(64), 0, st, t,
+                             ctx->d_sets, ctx->d_status);
+        else if (l.width == kLinear + 32)
+          hipLaunchKernelGGL(btpm_conduct_smooth_lin<2>, dim3(l.n), dim3(64), 0, st, t,
+                             ctx->d_sets, ctx->d_status);
+        else if (l.width == kLinear + 64)
+          hipLaunchKernelGGL(btpm_conduct_smooth_lin<4>, dim3(l.n), dim3(64), 0, st, t,
+                             ctx->d_sets, ctx->d_status);
+        else if (l.width == 64)
           hipLaunchKernelGGL(btpm_conduct_smooth<64>, dim3(l.n), dim3(64), 0, st, t,
                              ctx->d_sets, ctx->d_status);
         else if (l.width == 128)
@@ -1134,11 +1199,18 @@ struct Sched {
         if (l.trial) trial_event(st, 1);
       }
     } else if (ph == 2) {
-      const int n = fast ? fn_tiles_c : n_tiles_c;
-      if (n)
-        hipLaunchKernelGGL(btpm_conduct_crater, dim3(n), dim3(BTPM_CRATER_THREADS), 0, st,
-                           (fast ? fd_tiles_c : d_tiles_c).as<btpm_tile>(), ctx->d_sets,
-                           ctx->d_status);
+      for (const TileList& l : fast ? fcrater : crater_lists) {
+        const btpm_tile* t = l.tiles->as<btpm_tile>();
+        auto launch = [&](auto kernel, int threads) {
+          hipLaunchKernelGGL(kernel, dim3(l.n), dim3(threads), 0, st, t, ctx->d_sets,
+                             ctx->d_status);
+        };
+        switch (l.width) {
+          case kLinear + 5: launch(btpm_conduct_crater_lin<5>, 512); break;
+          case kLinear + 2: launch(btpm_conduct_crater_lin<2>, 256); break;
+          default: launch(btpm_conduct_crater, BTPM_CRATER_THREADS);
+        }
+      }
     } else {
       const int n = fast ? fn_ids : n_ids;
       if (n)
@@ -1563,11 +1635,16 @@ int btpm_shape_create(btpm_ctx* ctx, const btpm_params* p, const btpm_body* body
   sh->h_numrevs.assign(nf, 1.0f);
   if (body->numrevs) sh->h_numrevs.assign(body->numrevs, body->numrevs + nf);
   for (int f = 0; f < nf; ++f) {  // explicit-scheme stability, as the kernels assume
-    const double dz = 8.0 / BTPM_NX;
-    const float r = (float)((2.0 * kPi * sh->h_numrevs[f] / nt) / (dz * dz));
+    const float r = ftcs_number(sh->h_numrevs[f], nt);
     if (!(r >= 0.0f && r <= (float)BTPM_R_MAX))
       return fail(BTPM_ERR_ARG, "facet %d: dtau/dz^2 = %.6g outside [0, %g] (FTCS stability "
                   "limit; raise ntau)", f, (double)r, BTPM_R_MAX);
+  }
+  if (std::all_of(sh->h_numrevs.begin(), sh->h_numrevs.end(),
+                  [&](float n) { return n == sh->h_numrevs[0]; })) {
+    std::vector<_Float16> op(BTPM_LIN_OP);
+    linear_operator(ftcs_number(sh->h_numrevs[0], nt), nt, op.data());
+    upload(sh->op, op.data(), op.size(), st);
   }
   std::vector<float> oma(nf);
   for (int f = 0; f < nf; ++f) oma[f] = 1.0f - sh->h_albedo[f];

@@ -40,6 +40,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include "btpm_device.h"
 #include "btpm_internal.h"
 
 namespace btpm_lin {
@@ -162,9 +163,9 @@ __device__ __forceinline__ void transpose4(float& x0, float& x1, float& x2, floa
   swap16(x2, x3);
 }
 
-// Surface slots <-> one column per lane.  64 columns (NT = 4): lane 16 t + c
-// takes the 8 surface values of column c of tile t.  16 columns (NT = 1):
-// every lane group takes all 8 values of its column.
+// Surface slots <-> one column per lane: lane group g takes the 8 surface
+// values of its column of tile g % NT (with NT = 4 every lane its own column,
+// with NT = 2 and 1 two and four lanes the same).
 __device__ __forceinline__ void surface_out(const float (&u)[4][16], float (&w)[8]) {
 #pragma unroll
   for (int q = 0; q < 2; ++q) {
@@ -185,6 +186,30 @@ __device__ __forceinline__ void surface_in(float (&u)[4][16], const float (&w)[8
     u[1][q] = x1;
     u[2][q] = x2;
     u[3][q] = x3;
+  }
+}
+__device__ __forceinline__ void surface_out(const float (&u)[2][16], float (&w)[8]) {
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    float a = u[0][q], b = u[1][q];
+    swap16(a, b);  // a: tiles 0, 1 from group 0, then from group 2; b: 1, then 3
+    float a2 = a, b2 = b;
+    swap32(a, a2);
+    swap32(b, b2);
+    w[q] = a;
+    w[2 + q] = b;
+    w[4 + q] = a2;
+    w[6 + q] = b2;
+  }
+}
+__device__ __forceinline__ void surface_in(float (&u)[2][16], const float (&w)[8]) {
+  const bool hi = (threadIdx.x & 32) != 0;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    float a = hi ? w[4 + q] : w[q], b = hi ? w[6 + q] : w[2 + q];
+    swap16(a, b);
+    u[0][q] = a;
+    u[1][q] = b;
   }
 }
 __device__ __forceinline__ void surface_out(const float (&u)[1][16], float (&w)[8]) {
@@ -208,6 +233,76 @@ __device__ __forceinline__ void surface_in(float (&u)[1][16], const float (&w)[8
     const float lo = (g & 1) ? w[2 + q] : w[q];
     const float hi = (g & 1) ? w[6 + q] : w[4 + q];
     u[0][q] = (g & 2) ? hi : lo;
+  }
+}
+
+// The surface balances of a block's 8 steps for one column per lane (or copies
+// of it).  In: w = base(1..8), tot = the absorbed flux of each step, tp = the
+// previous rotation's surface temperatures; out: w = the surface offset before
+// each step (x 2^15), tp = this rotation's temperatures.
+//
+// The Newton start of a step is the previous rotation's temperature at this
+// step shifted by the difference between the two rotations, extrapolated
+// linearly from the steps two and three back.  Taking it from there rather
+// than from the step just solved leaves only
+//   u0 -> node 1 -> first iterate
+// (six dependent operations) between consecutive steps: the derivative, its
+// reciprocal and the start's residual are formed during the step before.  The
+// start only decides how many iterations a column takes, never where it stops.
+struct Surface {
+  float u0;           // surface offset x 2^15
+  float d1, d2, d3;   // T - T_prev one, two and three steps back
+  float dm;           // max |T - T_prev| of the rotation
+};
+
+// beside(k) is work of the caller's that does not depend on the steps, placed
+// beside step k.
+template <bool FULL, class Beside>
+__device__ __forceinline__ void surface_steps(Surface& s, float (&w)[8], float (&tp)[8],
+                                              const float (&tot)[8], const float (&gain)[8],
+                                              double m1, double es, double Tref, double tol, int cap,
+                                              int kend, Beside beside) {
+  // constants held in registers: as literals they cost a move at every use
+  double up = (double)kScale, down = 1.0 / (double)kScale;
+  asm volatile("" : "+s"(up), "+s"(down));
+  const double Trefs = -Tref * up;  // exact: a power of two
+  auto start = [&](int k, float a, float b) {  // a, b: differences two and three steps back
+    btpm_dev::FirstIterate f = btpm_dev::newton_first(
+        (double)(tp[k] + (3.0f * a - 2.0f * b)), (double)tot[k], m1, es);
+    return f;
+  };
+  btpm_dev::FirstIterate f = start(0, s.d2, s.d3);
+#pragma unroll
+  for (int k = 0; k < BTPM_BLK; ++k) {
+    if (!FULL && k >= kend) {
+      w[k] = 0.0f;
+      continue;
+    }
+    beside(k);
+#pragma unroll
+    for (int kk = k; kk < BTPM_BLK; ++kk) w[kk] = fmaf(gain[kk - k], s.u0, w[kk]);
+    const double t1 = fma((double)w[k], down, Tref);
+    w[k] = s.u0;  // the surface value before this step, an input of the product
+    double x = fma(f.b, t1, f.a);
+    const double d0 = x - f.x0;
+    btpm_dev::FirstIterate next = f;
+    if (k + 1 < BTPM_BLK) {
+      next = start(k + 1, s.d1, s.d2);
+      // formed here, beside this step's chain, not behind the branch below
+      asm volatile("" : "+v"(next.x0), "+v"(next.a), "+v"(next.b));
+#pragma unroll
+      for (int kk = k + 1; kk < BTPM_BLK; ++kk) asm volatile("" : "+v"(w[kk]));
+    }
+    if (__builtin_expect(__ballot(!(fabs(d0) < tol)) != 0, 0))  // a column needs another iteration
+      x = btpm_dev::newton_finish(fma(m1, t1, (double)tot[k]), m1, es, x, d0, tol, cap);
+    f = next;
+    s.u0 = (float)fma(x, up, Trefs);
+    const float t = (float)x;
+    s.d3 = s.d2;
+    s.d2 = s.d1;
+    s.d1 = t - tp[k];
+    s.dm = fmaxf(s.dm, fabsf(s.d1));
+    tp[k] = t;
   }
 }
 

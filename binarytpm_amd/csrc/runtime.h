@@ -156,6 +156,10 @@ void upload(DBuf& b, const T* h, size_t count, hipStream_t st) {
   }
 }
 
+// The 8-step conduction operator of FTCS number r over cycles of ntau steps
+// (linear_block.h) into op[BTPM_LIN_OP] (linear_op.hip).
+void linear_operator(float r, int ntau, _Float16* op);
+
 // VF^T as fp16 hi/lo tiles [2][112][112] (A[m=j][k=i] = vf[i*100+j]), zero
 // padded, scaled by 2^s so the largest entry lies in [0.5, 1): the low
 // halves then stay normal fp16 numbers.  Returns 2^-s.

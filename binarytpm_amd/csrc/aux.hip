@@ -112,26 +112,49 @@ extern "C" __global__ void btpm_unpack_crater_rows(const float* __restrict__ in,
 
 // initialisetemperatures, T175706/thermal.cpp:1861-1889, from the absorbed
 // flux src = (1-A)F (blocked):  T = (mean_s src / es)^(1/4) everywhere.
-extern "C" __global__ void btpm_init_smooth(btpm_set_dev S) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= S.ncols) return;
+// Workgroup: 8 columns x 32 lanes, a lane taking every 32nd time block of its
+// column (the 8 columns of a block are one 256-byte run), its FP64 partial
+// sums combined in lane order.  One lane per column waited for every block in
+// turn: 5120 columns of 650 steps 101 us, 1600 of 9750 steps 2.78 ms.
+extern "C" __global__ __launch_bounds__(256) void btpm_init_smooth(btpm_set_dev S) {
+  constexpr int kCols = 8, kParts = 32;
+  __shared__ double part[kParts][kCols];
+  const int lc = threadIdx.x % kCols, p = threadIdx.x / kCols;
+  const int c = min(blockIdx.x * kCols + lc, (unsigned)S.ncols - 1u);
+  const bool ok = blockIdx.x * kCols + lc < (unsigned)S.ncols;
   double sum = 0.0;
-  for (int b = 0; b < S.nb; ++b) {
-    const float* p = S.src + ((size_t)b * S.ncols + c) * BTPM_BLK;
+  for (int b = p; b < S.nb; b += kParts) {
+    const float4* v = reinterpret_cast<const float4*>(S.src + ((size_t)b * S.ncols + c) * BTPM_BLK);
+    const float4 x = v[0], y = v[1];
+    const float e[BTPM_BLK] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
     const int kend = min(BTPM_BLK, S.ntau - b * BTPM_BLK);
-    for (int k = 0; k < kend; ++k) sum += (double)p[k];
+#pragma unroll
+    for (int k = 0; k < BTPM_BLK; ++k)
+      if (k < kend) sum += (double)e[k];
   }
+  part[p][lc] = sum;
+  __syncthreads();
+  sum = 0.0;
+  for (int q = 0; q < kParts; ++q) sum += part[q][lc];
+  if (!ok) return;
   const float t = (float)pow(sum / S.ntau / (double)S.es, 0.25);
-  for (int i = 0; i < BTPM_PSTRIDE; ++i) S.prof[(size_t)c * BTPM_PSTRIDE + i] = t;
+  const float4 t4 = make_float4(t, t, t, t);
   const float e = S.esia * t * t * t * t;
-  for (int b = 0; b < S.nb; ++b) {
-    float* p = S.T + ((size_t)b * S.ncols + c) * BTPM_BLK;
-    for (int k = 0; k < BTPM_BLK; ++k) p[k] = t;
+  const float4 e4 = make_float4(e, e, e, e);
+  for (int i = p; i < BTPM_PSTRIDE / 4; i += kParts)
+    reinterpret_cast<float4*>(S.prof + (size_t)c * BTPM_PSTRIDE)[i] = t4;
+  for (int b = p; b < S.nb; b += kParts) {
+    float4* v = reinterpret_cast<float4*>(S.T + ((size_t)b * S.ncols + c) * BTPM_BLK);
+    v[0] = t4;
+    v[1] = t4;
   }
   if (S.emis)  // facet-major [c][nb*BLK]
-    for (int k = 0; k < S.nb * BTPM_BLK; ++k) S.emis[(size_t)c * S.nb * BTPM_BLK + k] = e;
-  S.frozen[c] = 0;
-  S.dmax[c] = 0.0f;
+    for (int i = p; i < S.nb * (BTPM_BLK / 4); i += kParts)
+      reinterpret_cast<float4*>(S.emis + (size_t)c * S.nb * BTPM_BLK)[i] = e4;
+  if (p == 0) {
+    S.frozen[c] = 0;
+    S.dmax[c] = 0.0f;
+  }
 }
 
 // Warm start of a smooth set whose T and profile were copied from a finished

@@ -698,16 +698,24 @@ struct Sched {
     return c;
   }
   // The operator's kernels (16, 32 or 64 columns per wave) share a launch, and
-  // what a width costs turns on how many waves all their sets make together:
-  // up to kLinCols columns every width leaves SIMDs without a wave, beyond it
-  // the copies of a column's balance compete, so the two are tuned apart.
-  static constexpr long long kLinCols = 32768;
+  // what a width costs turns on how many waves all their sets make together.
+  // Measured per 650-step rotation at 16 / 32 / 64: 5120 columns 101 / 121 /
+  // 163 us, 20480 columns 123 / 125 / 165 us, 40960 columns 156 / 154 / 170 us,
+  // 81920 columns 222 / 206 / 217 us: 16 up to kLinCols columns, 32 beyond.
+  // A trial runs in the first rotations, whose extra Newton iterations favour
+  // wide waves, so another width must be kLinMargin cheaper there.
+  static constexpr long long kLinCols = 20480;
+  static constexpr double kLinMargin = 0.10;
   TuneKey smooth_key(const SetHost* S) const {
     const long long c = log2_class(S->d.ncols);
     return S->d.op ? TuneKey{2, c | (linear_cols() > kLinCols ? 64 : 0)} : TuneKey{0, c};
   }
-  static std::vector<int> smooth_candidates(const SetHost* S) {
-    return S->d.op ? std::vector<int>{16, 32, 64} : std::vector<int>{256, 128, 64};
+  int smooth_default(const SetHost* S) const {
+    return S->d.op ? (linear_cols() > kLinCols ? 32 : 16) : BTPM_SMOOTH_WG;
+  }
+  std::vector<int> smooth_candidates(const SetHost* S) const {
+    if (!S->d.op) return {256, 128, 64};
+    return smooth_default(S) == 16 ? std::vector<int>{16, 32, 64} : std::vector<int>{32, 16, 64};
   }
   // Craters per workgroup of the operator's crater conduction, for all such
   // sets of a rotation together: 2 while every workgroup has a CU to itself
@@ -721,9 +729,6 @@ struct Sched {
       if (S->d.kind == BTPM_SET_CRATER && S->d.op) n += ctx->h_status[S->slot].norder;
     }
     return n <= kPairCraters ? 2 : 5;
-  }
-  int smooth_default(const SetHost* S) const {
-    return S->d.op ? (linear_cols() > kLinCols ? 64 : 16) : BTPM_SMOOTH_WG;
   }
   static TuneKey heat_key(const btpm_shape* sh) {
     return {1, (log2_class(sh->nnz) << 40) | (log2_class(sh->nf) << 24) | sh->nb};
@@ -777,7 +782,8 @@ struct Sched {
       // kept unless another is at least kTuneMargin cheaper: near-ties are
       // timing noise, and a decision flipped by noise carries over to every
       // later batch and server on the context
-      if (best != 0 && t.cost[best] / t.n[best] > (1.0 - kTuneMargin) * (t.cost[0] / t.n[0]))
+      const double margin = t.key.first == 2 ? kLinMargin : kTuneMargin;
+      if (best != 0 && t.cost[best] / t.n[best] > (1.0 - margin) * (t.cost[0] / t.n[0]))
         best = 0;
       ctx->tuned[t.key] = t.cand[best];
       stats.tune_decisions++;

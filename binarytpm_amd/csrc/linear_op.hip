@@ -23,14 +23,19 @@ int slot_entry(int g, int q) {
   return n <= N ? n - 1 : -1;
 }
 
-// one FTCS step of the nodes with surface value s (node 0) and the zero-flux
-// bottom u[NX] = u[NX-1]
-void ftcs(double (&u)[N], double r, double s) {
-  double before = s;
+// u[node - 1][entry]: the nodes as functions of the entries
+using Nodes = double[N][L];
+
+// one FTCS step of the nodes, entry by entry, with surface value s[entry]
+// (node 0) and the zero-flux bottom u[NX] = u[NX-1]
+void ftcs(Nodes& u, double r, const double (&s)[L]) {
+  double before[L], cur[L];
+  std::memcpy(before, s, sizeof before);
   for (int i = 0; i < N; ++i) {
-    const double cur = u[i], next = i + 1 < N ? u[i + 1] : cur;
-    u[i] = cur + r * (next - 2.0 * cur + before);
-    before = cur;
+    std::memcpy(cur, u[i], sizeof cur);
+    const double* next = i + 1 < N ? u[i + 1] : cur;
+    for (int e = 0; e < L; ++e) u[i][e] = cur[e] + r * (next[e] - 2.0 * cur[e] + before[e]);
+    std::memcpy(before, cur, sizeof before);
   }
 }
 
@@ -38,35 +43,37 @@ void ftcs(double (&u)[N], double r, double s) {
 // node 1 after 1..8 further steps without surface input
 void respond(double r, int steps, bool responses, double (&out)[L][L]) {
   std::memset(out, 0, sizeof out);
-  for (int e = 0; e < L; ++e) {
-    double u[N] = {0.0};
-    if (e < N) u[e] = 1.0;
-    for (int k = 0; k < steps; ++k) ftcs(u, r, e == N + k ? 1.0 : 0.0);
-    for (int i = 0; i < N; ++i) out[i][e] = u[i];
-    if (!responses) continue;
-    for (int s = 0; s < B; ++s) {
-      ftcs(u, r, 0.0);
-      out[N + s][e] = u[0];
-    }
+  Nodes u = {};
+  for (int i = 0; i < N; ++i) u[i][i] = 1.0;
+  for (int k = 0; k < steps; ++k) {
+    double s[L] = {0.0};
+    s[N + k] = 1.0;
+    ftcs(u, r, s);
+  }
+  std::memcpy(out, u, sizeof u);
+  if (!responses) return;
+  const double none[L] = {0.0};
+  for (int s = 0; s < B; ++s) {
+    ftcs(u, r, none);
+    std::memcpy(out[N + s], u[0], sizeof u[0]);
   }
 }
 
 // hi and lo of every entry times 2^15, the rounding of the low halves carried
 // along the row from its largest entry to its smallest
 void split_rows(const double (&m)[L][L], _Float16 (&hi)[L][L], _Float16 (&lo)[L][L]) {
+  std::memset(hi, 0, sizeof hi);
+  std::memset(lo, 0, sizeof lo);
   for (int i = 0; i < L; ++i) {
-    int by[L];
-    for (int j = 0; j < L; ++j) by[j] = j;
-    std::sort(by, by + L, [&](int a, int b) { return std::fabs(m[i][a]) > std::fabs(m[i][b]); });
+    int by[L], n = 0;
+    for (int j = 0; j < L; ++j)
+      if (m[i][j] != 0.0) by[n++] = j;
+    std::sort(by, by + n, [&](int a, int b) { return std::fabs(m[i][a]) > std::fabs(m[i][b]); });
     double carry = 0.0;
-    for (int k = 0; k < L; ++k) {
+    for (int k = 0; k < n; ++k) {
       const int j = by[k];
       const double x = m[i][j] * btpm_lin::kScale;
       hi[i][j] = (_Float16)x;
-      if (m[i][j] == 0.0) {
-        lo[i][j] = (_Float16)0.0f;
-        continue;
-      }
       const double w = x - (double)hi[i][j] + carry;
       lo[i][j] = (_Float16)w;
       carry = w - (double)lo[i][j];
@@ -102,16 +109,17 @@ void linear_operator(float rf, int ntau, _Float16* op) {
     pack(hi, lo, btpm_lin::kBlkTile[b], btpm_lin::kBlkChunk[b], op + btpm_lin::kTail + 2 * b * btpm_lin::kFrag);
   // base(1..8) of the first block from the nodes (no steps before it)
   respond(r, 0, true, m);
-  for (int i = 0; i < N; ++i)
-    for (int j = 0; j < L; ++j) m[i][j] = 0.0;
+  std::memset(m, 0, N * sizeof m[0]);
   split_rows(m, hi, lo);
   pack(hi, lo, 0, 0, op + btpm_lin::kInit);
   // g(k): node 1, k + 1 steps after a unit surface value
   float g[B];
-  double u[N] = {0.0};
+  Nodes u = {};
   for (int k = 0; k < B; ++k) {
-    ftcs(u, r, k == 0 ? 1.0 : 0.0);
-    g[k] = (float)u[0];
+    double x[L] = {0.0};
+    x[0] = k == 0 ? 1.0 : 0.0;
+    ftcs(u, r, x);
+    g[k] = (float)u[0][0];
   }
   std::memcpy(op + btpm_lin::kGain, g, sizeof g);
 }

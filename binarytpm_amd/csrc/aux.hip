@@ -1244,67 +1244,75 @@ extern "C" __global__ void btpm_finish_scatter(float* __restrict__ F, const floa
 }
 
 // ---------------------------------------------------------------------------
-// per-set status after a rotation (one workgroup per set)
+// per-set status after a rotation (one workgroup per set): sums of the tiles'
+// counts, the rotation count, and the stable compaction of the groups still
+// integrating into order[] for the next rotation.  1024 groups a pass: a
+// lane's place is its wave's ballot below it plus the counts of the waves
+// before (256 lanes with a scan in LDS of 16 barriers: 23 us for 5120 groups).
 // ---------------------------------------------------------------------------
-extern "C" __global__ __launch_bounds__(256) void btpm_status_kernel(
+extern "C" __global__ __launch_bounds__(1024) void btpm_status_kernel(
     const int* __restrict__ set_ids, const btpm_set_dev* __restrict__ sets,
     btpm_status_dev* __restrict__ status) {
-  __shared__ long long red_w[256];
-  __shared__ int red_a[256];
-  __shared__ int scan[256];
+  __shared__ long long red_w[16];
+  __shared__ int red_a[16];
+  __shared__ int count[2][16];
   const int sid = set_ids[blockIdx.x];
   const btpm_set_dev& S = sets[sid];
   btpm_status_dev* st = status + sid;
   if (st->done) return;
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // the tiles this rotation could fill: every launch list covers them and
   // each of their workgroups wrote its counts (later tiles may be stale)
   const int ntl = min(S.ntiles, (st->norder + S.tile_cols - 1) / S.tile_cols);
   long long w = 0;
   int a = 0;
-  for (int t = threadIdx.x; t < ntl; t += 256) {
+  for (int t = tid; t < ntl; t += 1024) {
     a += S.tile_active[t];
     w += S.tile_work[t];
   }
-  red_w[threadIdx.x] = w;
-  red_a[threadIdx.x] = a;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) {
-      red_w[threadIdx.x] += red_w[threadIdx.x + s];
-      red_a[threadIdx.x] += red_a[threadIdx.x + s];
-    }
-    __syncthreads();
+  for (int o = 32; o > 0; o >>= 1) {
+    a += __shfl_xor(a, o);
+    w += __shfl_xor(w, o);
   }
-  if (threadIdx.x == 0) {
+  if (lane == 0) {
+    red_w[wave] = w;
+    red_a[wave] = a;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    for (int i = 1; i < 16; ++i) {
+      a += red_a[i];
+      w += red_w[i];
+    }
     const int rev = st->rev;          // index of the rotation just executed
-    st->active = red_a[0];
-    st->colsteps += red_w[0] * (long long)S.ntau;
+    st->active = a;
+    st->colsteps += w * (long long)S.ntau;
     st->rev = rev + 1;
-    if (rev > S.check_after && red_a[0] == 0) {
+    if (rev > S.check_after && a == 0) {
       st->done = 1;
       st->converged = 1;
     } else if (rev + 1 >= S.max_rev) {
       st->done = 1;
     }
   }
-  // stable compaction of the groups still integrating into order[] for the
-  // next rotation (chunks of 256 with a block-wide inclusive scan)
-  const int tid = (int)threadIdx.x;
-  int base = 0;
-  for (int g0 = 0; g0 < S.ngroups; g0 += 256) {
+  const uint8_t* __restrict__ frozen = S.frozen;
+  int* __restrict__ order = S.order;
+  int base = 0, par = 0;
+  for (int g0 = 0; g0 < S.ngroups; g0 += 1024) {
     const int g = g0 + tid;
-    const int live = (g < S.ngroups && !S.frozen[g]) ? 1 : 0;
-    __syncthreads();  // the previous chunk's scan[255] has been read
-    scan[tid] = live;
+    const bool live = g < S.ngroups && !frozen[g];
+    const unsigned long long b = __ballot(live);
+    if (lane == 0) count[par][wave] = __popcll(b);
     __syncthreads();
-    for (int off = 1; off < 256; off <<= 1) {
-      const int v = tid >= off ? scan[tid - off] : 0;
-      __syncthreads();
-      scan[tid] += v;
-      __syncthreads();
+    int before = 0, all = 0;
+    for (int v = 0; v < 16; ++v) {
+      const int n = count[par][v];
+      before += v < wave ? n : 0;
+      all += n;
     }
-    if (live) S.order[base + scan[tid] - 1] = g;
-    base += scan[255];
+    if (live) order[base + before + __popcll(b & ((1ull << lane) - 1ull))] = g;
+    base += all;
+    par ^= 1;  // the next pass writes the other counts while slow waves read these
   }
   if (tid == 0) st->norder = base;
 }

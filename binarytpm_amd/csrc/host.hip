@@ -1220,7 +1220,7 @@ struct Sched {
     } else {
       const int n = fast ? fn_ids : n_ids;
       if (n)
-        hipLaunchKernelGGL(btpm_status_kernel, dim3(n), dim3(256), 0, st,
+        hipLaunchKernelGGL(btpm_status_kernel, dim3(n), dim3(1024), 0, st,
                            (fast ? fd_ids : d_ids).as<int>(), ctx->d_sets, ctx->d_status);
     }
   }

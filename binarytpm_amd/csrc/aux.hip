@@ -1246,9 +1246,11 @@ extern "C" __global__ void btpm_finish_scatter(float* __restrict__ F, const floa
 // ---------------------------------------------------------------------------
 // per-set status after a rotation (one workgroup per set): sums of the tiles'
 // counts, the rotation count, and the stable compaction of the groups still
-// integrating into order[] for the next rotation.  1024 groups a pass: a
-// lane's place is its wave's ballot below it plus the counts of the waves
-// before (256 lanes with a scan in LDS of 16 barriers: 23 us for 5120 groups).
+// integrating into order[] for the next rotation, class by class (perm lists
+// the groups by class), each class padded with -1 to whole tiles.  1024 groups
+// a pass: a lane's place is its wave's ballot below it plus the counts of the
+// waves before (256 lanes with a scan in LDS of 16 barriers: 23 us for 5120
+// groups).
 // ---------------------------------------------------------------------------
 extern "C" __global__ __launch_bounds__(1024) void btpm_status_kernel(
     const int* __restrict__ set_ids, const btpm_set_dev* __restrict__ sets,
@@ -1296,23 +1298,34 @@ extern "C" __global__ __launch_bounds__(1024) void btpm_status_kernel(
     }
   }
   const uint8_t* __restrict__ frozen = S.frozen;
+  const int* __restrict__ perm = S.perm;
   int* __restrict__ order = S.order;
   int base = 0, par = 0;
-  for (int g0 = 0; g0 < S.ngroups; g0 += 1024) {
-    const int g = g0 + tid;
-    const bool live = g < S.ngroups && !frozen[g];
-    const unsigned long long b = __ballot(live);
-    if (lane == 0) count[par][wave] = __popcll(b);
-    __syncthreads();
-    int before = 0, all = 0;
-    for (int v = 0; v < 16; ++v) {
-      const int n = count[par][v];
-      before += v < wave ? n : 0;
-      all += n;
+  for (int k = 0, g0 = 0; k < S.ncls; ++k) {
+    const int end = S.cls_end[k];
+    for (; g0 < end; g0 += 1024) {
+      const int i = g0 + tid;
+      const int g = i < end ? (perm ? perm[i] : i) : 0;
+      const bool live = i < end && !frozen[g];
+      const unsigned long long b = __ballot(live);
+      if (lane == 0) count[par][wave] = __popcll(b);
+      __syncthreads();
+      int before = 0, all = 0;
+      for (int v = 0; v < 16; ++v) {
+        const int n = count[par][v];
+        before += v < wave ? n : 0;
+        all += n;
+      }
+      if (live) order[base + before + __popcll(b & ((1ull << lane) - 1ull))] = g;
+      base += all;
+      par ^= 1;  // the next pass writes the other counts while slow waves read these
     }
-    if (live) order[base + before + __popcll(b & ((1ull << lane) - 1ull))] = g;
-    base += all;
-    par ^= 1;  // the next pass writes the other counts while slow waves read these
+    g0 = end;
+    if (S.ncls > 1) {
+      const int pad = (base + S.cls_pad - 1) / S.cls_pad * S.cls_pad;
+      for (int i = base + tid; i < pad; i += 1024) order[i] = -1;
+      base = pad;
+    }
   }
   if (tid == 0) st->norder = base;
 }

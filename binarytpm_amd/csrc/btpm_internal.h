@@ -55,6 +55,8 @@
 // halves of one 8-step conduction operator (linear_block.h): 12 + 12 + 2
 // matrix fragments of 512 halves and 8 floats, padded to 256 bytes
 #define BTPM_LIN_OP (26 * 512 + 128)
+// most FTCS numbers (spin rates) in one shape for which operators are kept
+#define BTPM_LIN_CLASSES 8
 // fewest columns per tile of the operator's smooth conduction kernels
 #define BTPM_LIN_MIN 16
 
@@ -84,8 +86,17 @@ struct btpm_set_dev {
   const float* r;     // [ngroups] FTCS number dtau/dz^2
   const float* m1;    // [ngroups] Gamma sqrt(2 pi n / P) / dz
   uint8_t* frozen;    // [ngroups]
-  int* order;         // [ngroups] groups to integrate; the status kernel compacts
-                      // the unfrozen ones to the front after every rotation
+  int* order;         // groups to integrate (-1: padding between classes); the status
+                      // kernel compacts the unfrozen ones to the front after every rotation
+  // Classes of groups by FTCS number, for the 8-step operator (others: one
+  // class): class k is perm[cls_end[k-1] .. cls_end[k]) (perm null: identity),
+  // its operator op + k BTPM_LIN_OP, its part of order[] padded to a multiple
+  // of cls_pad so that a tile holds one class.
+  int ncls;
+  int cls_pad;
+  int cls_end[BTPM_LIN_CLASSES];
+  const int* perm;
+  const uint8_t* cls; // [ngroups] class of a group (null: all 0)
   float* dmax;        // [ngroups] max |dT| of the last executed rotation
   float* qext;        // [nb][ncols][BLK] total flux incl. facet self-heating (or null)
   float* emis;        // [ncols][nb*BLK] esia T^4 for the next rotation (or null),

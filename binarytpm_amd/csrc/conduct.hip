@@ -369,7 +369,7 @@ template __global__ void btpm_conduct_smooth<64>(const btpm_tile*, const btpm_se
                                                  const btpm_status_dev*);
 
 // ---------------------------------------------------------------------------
-// Smooth facets with one FTCS number for the whole set, on the matrix cores
+// Smooth facets with at most BTPM_LIN_CLASSES FTCS numbers, on the matrix cores
 // (linear_block.h): one wave per workgroup, 16 NT columns.  NT = 1, 2: four
 // or two lanes solve the surface balances of the same column (the balance is a
 // chain of dependent FP64 operations, so the copies cost no time where a SIMD
@@ -391,10 +391,16 @@ __global__ __launch_bounds__(64, 2) void btpm_conduct_smooth_lin(
   const bool check = st.rev > S.check_after;
   const int lane = (int)threadIdx.x, g = lane >> 4;
   const int ncols = S.ncols, norder = st.norder;
-  const int last = norder > 0 ? norder - 1 : 0;
-  const int idx = tl.tile * W + lane % W;
-  const bool valid = idx < norder;
-  const int c = S.order[valid ? idx : last];
+  // lane -> column through the compacted order; a tile holds columns of one
+  // class, lanes past its columns mirror the first
+  const int first = tl.tile * W < norder ? S.order[tl.tile * W] : -1;
+  auto tile_col = [&](int l) {
+    const int i = tl.tile * W + l;
+    return i < norder ? S.order[i] : -1;
+  };
+  const int own = tile_col(lane % W);
+  const bool valid = own >= 0;
+  const int c = max(valid ? own : first, 0);
   const bool active = valid && (S.inst || !S.frozen[c]);
   const bool mine = active && lane < W;  // the lane that stores the column
   const int nwork = __popcll(__ballot(mine));
@@ -451,23 +457,22 @@ __global__ __launch_bounds__(64, 2) void btpm_conduct_smooth_lin(
       store_block(b, out);
     }
   } else {
-    const GLOBAL_AS h8* __restrict__ op = (const GLOBAL_AS h8*)S.op + lane;
+    const _Float16* opk = static_cast<const _Float16*>(S.op) +
+                          (S.cls != nullptr ? (size_t)S.cls[first] * BTPM_LIN_OP : 0);
+    const GLOBAL_AS h8* __restrict__ op = (const GLOBAL_AS h8*)opk + lane;
     h8 A[kFrags];
 #pragma unroll
     for (int i = 0; i < kFrags; ++i) A[i] = op[i * 64];
     float gain[BTPM_BLK];
 #pragma unroll
     for (int k = 0; k < BTPM_BLK; ++k)
-      gain[k] = reinterpret_cast<const float*>(static_cast<const _Float16*>(S.op) + kGain)[k];
+      gain[k] = reinterpret_cast<const float*>(opk + kGain)[k];
     const gfloat* prof = (const gfloat*)S.prof;
-    auto tile_col = [&](int t) {
-      const int i = tl.tile * W + 16 * t + (lane & 15);
-      return S.order[i < norder ? i : last];
-    };
     float u[NT][16];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      const gfloat* rec = prof + (size_t)tile_col(t) * BTPM_PSTRIDE;
+      const int ct = tile_col(16 * t + (lane & 15));
+      const gfloat* rec = prof + (size_t)(ct >= 0 ? ct : first) * BTPM_PSTRIDE;
       load_nodes(rec, g, rec[NX], u[t]);
     }
     const gfloat* rec = prof + (size_t)c * BTPM_PSTRIDE;
@@ -506,8 +511,8 @@ __global__ __launch_bounds__(64, 2) void btpm_conduct_smooth_lin(
 
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      const int ct = tile_col(t);
-      if (tl.tile * W + 16 * t + (lane & 15) >= norder || S.frozen[ct]) continue;
+      const int ct = tile_col(16 * t + (lane & 15));
+      if (ct < 0 || S.frozen[ct]) continue;
       gfloat* r = (gfloat*)S.prof + (size_t)ct * BTPM_PSTRIDE;
       store_nodes(r, g, r[NX], u[t]);
     }
@@ -933,7 +938,7 @@ extern "C" __global__ __launch_bounds__(BTPM_CRATER_THREADS) void btpm_conduct_c
 }
 
 // ---------------------------------------------------------------------------
-// Crater columns with one FTCS number for the whole set, on the 8-step
+// Crater columns of at most BTPM_LIN_CLASSES FTCS numbers, on the 8-step
 // operator (linear_block.h): P craters x 100 sub-facets per workgroup, lane ->
 // column in the surface steps, four 16-column tiles per wave in the operator's
 // product.  The crater product of block b + 1 needs only the previous
@@ -1054,19 +1059,18 @@ __global__ __launch_bounds__((P * BTPM_NS + 63) / 64 * 64) void btpm_conduct_cra
   const int tid = (int)threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g4 = lane >> 4;
   const int norder = st.norder;
-  const int last = norder > 0 ? norder - 1 : 0;
-  // local column -> column through the compacted order; idle lanes and slots
-  // past its end mirror a valid crater's column
-  auto column = [&](int lcol) {
-    const int l = lcol < P * NS ? lcol : P * NS - 1;
-    const int slot = tl.tile * P + l / NS;
-    return S.order[slot < norder ? slot : last] * NS + l % NS;
+  // local crater -> crater through the compacted order (a tile holds craters
+  // of one class); idle lanes and empty slots mirror the first crater's columns
+  const int first = tl.tile * P < norder ? S.order[tl.tile * P] : -1;
+  auto crater = [&](int l) {
+    const int slot = tl.tile * P + l;
+    return l < P && slot < norder ? S.order[slot] : -1;
   };
-  const int lc = tid < P * NS ? tid : P * NS - 1;
-  const int lcr = lc / NS, j = lc - lcr * NS;
-  const int c = column(tid);
-  const int gr = c / NS;
-  const bool active = tid < P * NS && tl.tile * P + lcr < norder && !S.frozen[gr];
+  const int lcr = tid / NS, j = tid % NS;
+  const int own = crater(lcr);
+  const int gr = max(own >= 0 ? own : first, 0);
+  const int c = gr * NS + j;
+  const bool active = own >= 0 && !S.frozen[gr];
   const int nwork = __syncthreads_count(active);
   if (nwork == 0) {
     if (tid == 0) {
@@ -1081,9 +1085,11 @@ __global__ __launch_bounds__((P * BTPM_NS + 63) / 64 * 64) void btpm_conduct_cra
   for (int e = tid; e < 4 * G::kBH; e += TH) (&lds_b[0][0])[e] = (_Float16)0.0f;
   if (tid >= P * NS)
     for (int k = 0; k < BTPM_BLK; ++k) lds_q[0][k * G::kQC + tid] = lds_q[1][k * G::kQC + tid] = 0.0f;
+  const _Float16* opk = static_cast<const _Float16*>(S.op) +
+                        (S.cls != nullptr ? (size_t)S.cls[first] * BTPM_LIN_OP : 0);
   if constexpr (G::kOpLds)
     for (int e = tid; e < kFrags * 64; e += TH)
-      reinterpret_cast<h8*>(lds_op)[e] = static_cast<const h8*>(S.op)[e];
+      reinterpret_cast<h8*>(lds_op)[e] = reinterpret_cast<const h8*>(opk)[e];
   VfFrag vf[G::kM];
 #pragma unroll
   for (int m = 0; m < G::kM; ++m)  // past the last m tile: any tile, its rows are not stored
@@ -1103,7 +1109,7 @@ __global__ __launch_bounds__((P * BTPM_NS + 63) / 64 * 64) void btpm_conduct_cra
   __syncthreads();  // the cleared E rows, the operator
 
   // emission of a block, fp16 hi / lo, into E buffer i (idle lanes: rows 8P..)
-  _Float16* const eb = &lds_b[0][(tid / NS * BTPM_BLK) * kLdsK + tid % NS];
+  _Float16* const eb = &lds_b[0][lcr * BTPM_BLK * kLdsK + j];
   auto split_e = [&](int i, const float (&t)[BTPM_BLK]) {
 #pragma unroll
     for (int k = 0; k < BTPM_BLK; ++k) {
@@ -1161,7 +1167,7 @@ __global__ __launch_bounds__((P * BTPM_NS + 63) / 64 * 64) void btpm_conduct_cra
       if (active) store8(Tout + (size_t)b * bstride, t);
     }
   } else {
-    const GLOBAL_AS h8* op = (const GLOBAL_AS h8*)S.op + lane;
+    const GLOBAL_AS h8* op = (const GLOBAL_AS h8*)opk + lane;
     const h8* lop = reinterpret_cast<const h8*>(lds_op) + lane;
     h8 A[G::kOpLds ? 1 : kFrags];
     if constexpr (!G::kOpLds)
@@ -1170,12 +1176,13 @@ __global__ __launch_bounds__((P * BTPM_NS + 63) / 64 * 64) void btpm_conduct_cra
     float gain[BTPM_BLK];
 #pragma unroll
     for (int k = 0; k < BTPM_BLK; ++k)
-      gain[k] = reinterpret_cast<const float*>(static_cast<const _Float16*>(S.op) + kGain)[k];
+      gain[k] = reinterpret_cast<const float*>(opk + kGain)[k];
     const gfloat* prof = (const gfloat*)S.prof;
     float u[4][16];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      const gfloat* rec = prof + (size_t)column(64 * wave + 16 * t + (lane & 15)) * BTPM_PSTRIDE;
+      const int l = 64 * wave + 16 * t + (lane & 15), ct = crater(l / NS);
+      const gfloat* rec = prof + (size_t)((ct >= 0 ? ct : first) * NS + l % NS) * BTPM_PSTRIDE;
       load_nodes(rec, g4, rec[NX], u[t]);
     }
     const gfloat* rec = prof + (size_t)c * BTPM_PSTRIDE;
@@ -1264,10 +1271,9 @@ __global__ __launch_bounds__((P * BTPM_NS + 63) / 64 * 64) void btpm_conduct_cra
 
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      const int l = 64 * wave + 16 * t + (lane & 15);
-      const int ct = column(l);
-      if (l >= P * NS || tl.tile * P + l / NS >= norder || S.frozen[ct / NS]) continue;
-      gfloat* r = (gfloat*)S.prof + (size_t)ct * BTPM_PSTRIDE;
+      const int l = 64 * wave + 16 * t + (lane & 15), ct = crater(l / NS);
+      if (ct < 0 || S.frozen[ct]) continue;
+      gfloat* r = (gfloat*)S.prof + (size_t)(ct * NS + l % NS) * BTPM_PSTRIDE;
       store_nodes(r, g4, r[NX], u[t]);
     }
     if (active) ((gfloat*)S.prof)[(size_t)c * BTPM_PSTRIDE] = fmaf(sf.u0, 1.0f / kScale, Tref);

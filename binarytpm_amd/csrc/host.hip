@@ -300,7 +300,11 @@ struct btpm_shape {
   // creation, then each solve's RGH; every use is on the context's stream)
   DBuf wfm;
   float vf_unscale = 1.0f;
-  DBuf op;  // 8-step conduction operator when every facet has one FTCS number
+  // 8-step conduction operators, one per FTCS number of the facets (empty with
+  // more than BTPM_LIN_CLASSES of them): the facets by class, the classes' ends,
+  // each facet's class (the last two empty with one class)
+  DBuf op, perm, cls;
+  std::vector<int> h_perm, cls_end;
   std::vector<float> h_albedo, h_numrevs;
 };
 
@@ -311,15 +315,30 @@ struct SetHost {
   int slot = -1;
   DBuf src, T, prof, r, m1, frozen, order, dmax, qext, emis, tile_active, tile_work;
   int ntiles = 0;
+  int norder = 0;  // entries of order[] at the start
   int listed = 0;  // tiles in the current launch lists
 };
 
-// order[] starts as the identity: every group integrates
-void alloc_order(SetHost* S, int ngroups, hipStream_t st) {
-  std::vector<int> id((size_t)ngroups);
-  for (int g = 0; g < ngroups; ++g) id[g] = g;
+// order[] starts with every group, class by class, each class padded to a
+// multiple of pad (one class: the identity)
+void alloc_order(SetHost* S, const btpm_shape* sh, int pad, hipStream_t st) {
+  btpm_set_dev& d = S->d;
+  const bool classes = d.op != nullptr && sh->cls_end.size() > 1;
+  d.ncls = classes ? (int)sh->cls_end.size() : 1;
+  d.cls_pad = pad;
+  d.cls_end[0] = d.ngroups;
+  if (classes) std::copy(sh->cls_end.begin(), sh->cls_end.end(), d.cls_end);
+  d.perm = classes ? sh->perm.as<int>() : nullptr;
+  d.cls = classes ? sh->cls.as<uint8_t>() : nullptr;
+  std::vector<int> id;
+  id.reserve((size_t)d.ngroups + (size_t)d.ncls * pad);
+  for (int k = 0, i = 0; k < d.ncls; ++k) {
+    for (; i < d.cls_end[k]; ++i) id.push_back(classes ? sh->h_perm[i] : i);
+    if (classes) id.resize((id.size() + pad - 1) / pad * pad, -1);
+  }
+  S->norder = (int)id.size();
   upload(S->order, id.data(), id.size(), st);
-  S->d.order = S->order.as<int>();
+  d.order = S->order.as<int>();
 }
 
 }  // namespace
@@ -434,15 +453,15 @@ void build_smooth(btpm_solve* s, hipStream_t st) {
   upload(S->r, r.data(), r.size(), st);
   upload(S->m1, m1.data(), m1.size(), st);
   S->frozen.alloc(d.ncols);
-  alloc_order(S.get(), d.ncols, st);
+  d.op = sh->op.p;
+  alloc_order(S.get(), sh, 64, st);  // 64: the widest tile
   S->dmax.alloc(d.ncols * sizeof(float));
   if (sh->nnz > 0) {
     S->qext.alloc(nser * sizeof(float));
     S->emis.alloc(nser * sizeof(float));
   }
   // tile arrays for the narrowest width
-  d.op = sh->op.p;
-  S->ntiles = d.op ? (d.ncols + BTPM_LIN_MIN - 1) / BTPM_LIN_MIN : (d.ncols + 63) / 64;
+  S->ntiles = d.op ? (S->norder + BTPM_LIN_MIN - 1) / BTPM_LIN_MIN : (d.ncols + 63) / 64;
   S->tile_active.alloc(S->ntiles * sizeof(int));
   S->tile_work.alloc(S->ntiles * sizeof(int));
   d.src = S->src.as<float>();
@@ -496,10 +515,10 @@ void build_crater(btpm_solve* s, hipStream_t st) {
   upload(S->r, r.data(), r.size(), st);
   upload(S->m1, m1.data(), m1.size(), st);
   S->frozen.alloc(d.ngroups);
-  alloc_order(S.get(), d.ngroups, st);
-  S->dmax.alloc(d.ngroups * sizeof(float));
   d.op = sh->op.p;
-  S->ntiles = d.op ? (d.ngroups + 1) / 2 : (d.ngroups + BTPM_CRATERS_WG - 1) / BTPM_CRATERS_WG;
+  alloc_order(S.get(), sh, 10, st);  // 10: whole tiles of 2 and of 5 craters
+  S->dmax.alloc(d.ngroups * sizeof(float));
+  S->ntiles = d.op ? (S->norder + 1) / 2 : (d.ngroups + BTPM_CRATERS_WG - 1) / BTPM_CRATERS_WG;
   S->tile_active.alloc(S->ntiles * sizeof(int));
   S->tile_work.alloc(S->ntiles * sizeof(int));
   d.src = S->src.as<float>();
@@ -877,7 +896,7 @@ struct Sched {
   void add_set(btpm_solve* s, SetHost* S) {
     S->slot = take_slot();
     btpm_status_dev z{};
-    z.norder = S->d.ngroups;
+    z.norder = S->norder;
     ctx->h_status[S->slot] = z;
     HIPCHK(hipMemcpyAsync(ctx->d_sets + S->slot, &S->d, sizeof(btpm_set_dev),
                           hipMemcpyHostToDevice, ctx->stream));
@@ -1646,11 +1665,29 @@ int btpm_shape_create(btpm_ctx* ctx, const btpm_params* p, const btpm_body* body
       return fail(BTPM_ERR_ARG, "facet %d: dtau/dz^2 = %.6g outside [0, %g] (FTCS stability "
                   "limit; raise ntau)", f, (double)r, BTPM_R_MAX);
   }
-  if (std::all_of(sh->h_numrevs.begin(), sh->h_numrevs.end(),
-                  [&](float n) { return n == sh->h_numrevs[0]; })) {
-    std::vector<_Float16> op(BTPM_LIN_OP);
-    linear_operator(ftcs_number(sh->h_numrevs[0], nt), nt, op.data());
-    upload(sh->op, op.data(), op.size(), st);
+  {
+    std::vector<float> rates;  // in order of first appearance
+    std::vector<uint8_t> cls(nf);
+    for (int f = 0; f < nf && rates.size() <= BTPM_LIN_CLASSES; ++f) {
+      size_t k = 0;
+      while (k < rates.size() && rates[k] != sh->h_numrevs[f]) ++k;
+      if (k == rates.size()) rates.push_back(sh->h_numrevs[f]);
+      cls[f] = (uint8_t)k;
+    }
+    if (rates.size() <= BTPM_LIN_CLASSES) {
+      std::vector<_Float16> op(rates.size() * BTPM_LIN_OP);
+      for (size_t k = 0; k < rates.size(); ++k) {
+        linear_operator(ftcs_number(rates[k], nt), nt, op.data() + k * BTPM_LIN_OP);
+        for (int f = 0; f < nf; ++f)
+          if (cls[f] == k) sh->h_perm.push_back(f);
+        sh->cls_end.push_back((int)sh->h_perm.size());
+      }
+      upload(sh->op, op.data(), op.size(), st);
+      if (rates.size() > 1) {
+        upload(sh->perm, sh->h_perm.data(), nf, st);
+        upload(sh->cls, cls.data(), nf, st);
+      }
+    }
   }
   std::vector<float> oma(nf);
   for (int f = 0; f < nf; ++f) oma[f] = 1.0f - sh->h_albedo[f];

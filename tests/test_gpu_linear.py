@@ -85,3 +85,44 @@ def test_widths_bitwise(ctx, rough80, ntau):
     for m in many:
         m.close()
     shape.close()
+
+
+@pytest.mark.parametrize("rates", [(0.5, 1.0), (1.0, 0.5, 0.25), tuple(np.linspace(0.25, 1.0, 8))])
+@pytest.mark.parametrize("nf", [9, 77])
+def test_spin_rate_classes_bitwise(ctx, rough80, rates, nf):
+    """Without exchange between facets, facets of several spin rates in one
+    shape equal the same facets in shapes of one rate each."""
+    case, crater = rough80
+    rng = np.random.default_rng(nf + len(rates))
+    pick = rng.integers(0, len(rates), nf)
+    p, _ = _fixed(650, case.rot_period, 8)
+    cm = th.CraterModel(vf=crater["vf"], solar=crater["solar"],
+                        shadow=crater["shadow"][:nf], cosang=crater["cosang"][:nf])
+    illum = case.illum[:nf]
+
+    def run(numrevs):
+        shape = th.Shape(ctx, p, illum, 0.1, numrevs=numrevs.astype(np.float32), crater=cm)
+        s = th.Solve(ctx, shape, 150.0, with_craters=True).run()
+        out = (s.surface_temps(), s.profile(), s.crater_temps(), s.crater_profile())
+        s.close()
+        shape.close()
+        return out
+
+    mixed = run(np.asarray(rates)[pick])
+    for k, r in enumerate(rates):
+        for m, u in zip(mixed, run(np.full(nf, r))):
+            assert np.array_equal(m[pick == k], u[pick == k])
+
+
+def test_many_spin_rates(ctx):
+    """More rates than operators are kept for."""
+    case = inputs.config0(subdiv=1, ntau=650)
+    nr = np.linspace(0.3, 1.0, 80).astype(np.float32)
+    p, po = _fixed(650, case.rot_period, 9)
+    shape = th.Shape(ctx, p, case.illum, 0.1, numrevs=nr)
+    s = th.Solve(ctx, shape, 150.0).run()
+    ref = O.smooth_solve(po, case.illum, 0.1, 150.0, numrevs=nr)
+    assert np.abs(s.surface_temps() - ref.stemp).max() <= TOL
+    assert np.abs(s.profile() - ref.temp).max() <= TOL
+    s.close()
+    shape.close()

@@ -341,12 +341,8 @@ extern "C" int btpm_geometry_illumination(btpm_ctx* ctx, const btpm_geometry* g,
                        sun_facet ? d_sun.as<float>() : nullptr);
     HIPCHK(hipGetLastError());
   }
-  HIPCHK(hipMemcpyAsync(shadow, d_shadow.p, nser * sizeof(int), hipMemcpyDeviceToHost, st));
-  if (illum)
-    HIPCHK(hipMemcpyAsync(illum, d_illum.p, nser * sizeof(float), hipMemcpyDeviceToHost, st));
-  if (sun_facet)
-    HIPCHK(hipMemcpyAsync(sun_facet, d_sun.p, 3 * nser * sizeof(float), hipMemcpyDeviceToHost,
-                          st));
-  HIPCHK(hipStreamSynchronize(st));
+  download_staged(ctx, shadow, d_shadow.p, nser * sizeof(int));
+  if (illum) download_staged(ctx, illum, d_illum.p, nser * sizeof(float));
+  if (sun_facet) download_staged(ctx, sun_facet, d_sun.p, 3 * nser * sizeof(float));
   API_END
 }

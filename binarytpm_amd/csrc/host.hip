@@ -1474,14 +1474,39 @@ struct Sched {
 // ===========================================================================
 namespace btpm {
 namespace {
-constexpr size_t kStageSlice = 256u << 20;
+// Copies between the device and pageable memory, in slices through two pinned
+// buffers.  Measured on 64 MB: to a host buffer of untouched 4 KB pages the
+// runtime's own copy reaches 3.9 GB/s (untouched 2 MB pages 10.8, a touched
+// buffer 7 to 18), since it takes the page faults on one thread; eight threads
+// behind the DMA reach 33 to 40.  From 4 MB on the staged copy is the faster
+// one down, and from 16 MB on up (64 MB: 37 GB/s against 47), where there is
+// nothing to fault in.  A quarter of the copy per slice keeps DMA and threads
+// both busy; slices of 2 MB lose the gain to starting the threads.
+constexpr size_t kStageSlice = 32u << 20, kStageSliceMin = 4u << 20;
+constexpr size_t kStageDown = 4u << 20, kStageUp = 16u << 20;
+
+size_t stage_slice(size_t bytes) {
+  const size_t quarter = ((bytes + 3) / 4 + 4095) & ~(size_t)4095;
+  return std::min(kStageSlice, std::max(kStageSliceMin, quarter));
+}
+
+// pinned host memory goes by DMA alone
+bool host_pinned(const void* p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type == hipMemoryTypeHost;
+}
 
 void stage_buffers(btpm_ctx* ctx) {
-  for (int k = 0; k < 2; ++k)
-    if (!ctx->stage[k]) {
+  for (int k = 0; k < 2; ++k) {
+    if (!ctx->stage[k])
       HIPCHK(hipHostMalloc((void**)&ctx->stage[k], kStageSlice, hipHostMallocDefault));
+    if (!ctx->stage_ev[k])
       HIPCHK(hipEventCreateWithFlags(&ctx->stage_ev[k], hipEventDisableTiming));
-    }
+  }
 }
 
 // memcpy split over up to 8 host threads (pageable <-> pinned slices)
@@ -1505,7 +1530,7 @@ void par_memcpy(char* d, const char* s, size_t n) {
 
 void upload_staged(btpm_ctx* ctx, void* dst, const void* src, size_t bytes) {
   hipStream_t st = ctx->stream;
-  if (bytes < 2 * kStageSlice) {
+  if (bytes < kStageUp || host_pinned(src)) {
     if (bytes) HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st));
     HIPCHK(hipStreamSynchronize(st));
     return;
@@ -1513,9 +1538,10 @@ void upload_staged(btpm_ctx* ctx, void* dst, const void* src, size_t bytes) {
   stage_buffers(ctx);
   const char* s = static_cast<const char*>(src);
   char* d = static_cast<char*>(dst);
+  const size_t slice = stage_slice(bytes);
   size_t i = 0;
-  for (size_t off = 0; off < bytes; off += kStageSlice, ++i) {
-    const size_t n = std::min(kStageSlice, bytes - off);
+  for (size_t off = 0; off < bytes; off += slice, ++i) {
+    const size_t n = std::min(slice, bytes - off);
     const int k = (int)(i & 1);
     // this buffer's previous slice has left for the device
     if (i >= 2) HIPCHK(hipEventSynchronize(ctx->stage_ev[k]));
@@ -1528,7 +1554,7 @@ void upload_staged(btpm_ctx* ctx, void* dst, const void* src, size_t bytes) {
 
 void download_staged(btpm_ctx* ctx, void* dst, const void* src, size_t bytes) {
   hipStream_t st = ctx->stream;
-  if (bytes < 2 * kStageSlice) {
+  if (bytes < kStageDown || host_pinned(dst)) {
     if (bytes) HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
     return;
@@ -1536,9 +1562,9 @@ void download_staged(btpm_ctx* ctx, void* dst, const void* src, size_t bytes) {
   stage_buffers(ctx);
   const char* s = static_cast<const char*>(src);
   char* d = static_cast<char*>(dst);
-  const size_t ns = (bytes + kStageSlice - 1) / kStageSlice;
+  const size_t slice = stage_slice(bytes), ns = (bytes + slice - 1) / slice;
   auto issue = [&](size_t j) {
-    const size_t off = j * kStageSlice, n = std::min(kStageSlice, bytes - off);
+    const size_t off = j * slice, n = std::min(slice, bytes - off);
     HIPCHK(hipMemcpyAsync(ctx->stage[j & 1], s + off, n, hipMemcpyDeviceToHost, st));
     HIPCHK(hipEventRecord(ctx->stage_ev[j & 1], st));
   };
@@ -1547,8 +1573,8 @@ void download_staged(btpm_ctx* ctx, void* dst, const void* src, size_t bytes) {
     // the other buffer's slice was copied out in the previous pass
     if (j + 1 < ns) issue(j + 1);
     HIPCHK(hipEventSynchronize(ctx->stage_ev[j & 1]));
-    const size_t off = j * kStageSlice;
-    par_memcpy(d + off, ctx->stage[j & 1], std::min(kStageSlice, bytes - off));
+    const size_t off = j * slice;
+    par_memcpy(d + off, ctx->stage[j & 1], std::min(slice, bytes - off));
   }
 }
 }  // namespace btpm
@@ -1858,7 +1884,7 @@ int btpm_shape_create(btpm_ctx* ctx, const btpm_params* p, const btpm_body* body
   const size_t nser = (size_t)nb * nf * BTPM_BLK;
   {
     DBuf raw;
-    upload(raw, body->illum, (size_t)nf * nt, st);
+    upload_big(ctx, raw, body->illum, (size_t)nf * nt);
     sh->F.alloc(nser * sizeof(float));
     hipLaunchKernelGGL(btpm_pack_blocked, dim3(grid1((size_t)nf * nb, 256)), dim3(256), 0, st,
                        raw.as<float>(), sh->F.as<float>(), (const float*)nullptr, nf, nt, nb);
@@ -1942,7 +1968,7 @@ int btpm_shape_create(btpm_ctx* ctx, const btpm_params* p, const btpm_body* body
       DBuf dsh, dcos, dsun, dvis, dnrm, rgi_blk, rgi;
       const bool by_sun = crater->sun_local != nullptr;
       if (by_sun) {  // shadow and cosine evaluated in the scattering kernel
-        upload(dsun, crater->sun_local, (size_t)nf * nt * 3, st);
+        upload_big(ctx, dsun, crater->sun_local, (size_t)nf * nt * 3);
         upload(dvis, crater->vis_table, (size_t)crater->n_el * crater->n_az * BTPM_NS, st);
         upload(dnrm, crater->normals, (size_t)BTPM_NS * 3, st);
       } else {
@@ -2005,8 +2031,7 @@ int btpm_shape_facet_illum(btpm_shape* sh, float* out) {
   raw.alloc((size_t)sh->nf * sh->p.ntau * 4);
   hipLaunchKernelGGL(btpm_unpack_blocked, dim3(grid1((size_t)sh->nf * sh->nb, 256)), dim3(256), 0,
                      c->stream, sh->F.as<float>(), raw.as<float>(), sh->nf, sh->p.ntau, sh->nb);
-  HIPCHK(hipMemcpyAsync(out, raw.p, raw.n, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  download_staged(c, out, raw.p, raw.n);
   API_END
 }
 
@@ -2022,8 +2047,7 @@ int btpm_shape_crater_illum(btpm_shape* sh, float* out) {
   hipLaunchKernelGGL(btpm_unpack_crater, dim3(grid1((size_t)sh->nf * BTPM_NS * sh->nb, 256)),
                      dim3(256), 0, c->stream, sh->cillum.as<float>(), raw.as<float>(), sh->nf,
                      sh->p.ntau, sh->nb);
-  HIPCHK(hipMemcpyAsync(out, raw.p, raw.n, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  download_staged(c, out, raw.p, raw.n);
   API_END
 }
 
@@ -2250,7 +2274,6 @@ static int fetch_series(btpm_solve* s, SetHost* S, float* out, int crater) {
   // large results leave through the context's pinned slices (host threads
   // copy one slice out while the DMA fills the other)
   download_staged(c, out, raw.p, raw.n);
-  HIPCHK(hipStreamSynchronize(c->stream));
   API_END
 }
 
@@ -2366,8 +2389,7 @@ static int fetch_profile(btpm_solve* s, SetHost* S, float* out, int crater) {
   HIPCHK(hipSetDevice(c->device));
   const int nc = S->d.ncols, np = BTPM_NX + 1;
   std::vector<float> h((size_t)BTPM_PSTRIDE * nc);
-  HIPCHK(hipMemcpyAsync(h.data(), S->prof.p, h.size() * 4, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  download_staged(c, h.data(), S->prof.p, h.size() * 4);
   // device [i][c] -> smooth [f][i], crater [f][i][j]
   if (!crater) {
     for (int f = 0; f < nc; ++f)

@@ -979,10 +979,8 @@ extern "C" int btpm_crater_sunlight(btpm_ctx* ctx, const btpm_crater_sun_in* in,
   d_co.alloc((size_t)first * ncf * sizeof(float));
   for (long long q0 = 0; q0 < total; q0 += chunk) {
     const long long n = std::min(chunk, total - q0);
-    HIPCHK(hipMemcpyAsync(d_lit.p, in->shadow + q0, (size_t)n * sizeof(int),
-                          hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(d_sun.p, in->sun + 3 * q0, (size_t)n * 3 * sizeof(float),
-                          hipMemcpyHostToDevice, st));
+    upload_staged(ctx, d_lit.p, in->shadow + q0, (size_t)n * sizeof(int));
+    upload_staged(ctx, d_sun.p, in->sun + 3 * q0, (size_t)n * 3 * sizeof(float));
     hipLaunchKernelGGL(btpm_crater_sun, dim3((unsigned)((n + 63) / 64)), dim3(256), shm, st,
                        d_lit.as<int>(), d_sun.as<float>(), d_cs.as<float4>(), d_samp.as<float4>(),
                        d_vt.as<float>(), ncf, nsamp, in->crater_radius, n, d_sh.as<float>(),

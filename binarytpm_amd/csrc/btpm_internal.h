@@ -33,7 +33,7 @@
 // halves per packed shape->crater view-factor tile: [hi, lo][112 sub-facets][32 entries]
 #define BTPM_DRF_TILE (2 * 112 * 32)
 // doubles per facet record of the shadow tests (geometry.hip)
-#define BTPM_GEOM_REC 20
+#define BTPM_GEOM_REC 18
 // floats per facet record of the view-factor producer (viewfactor.hip)
 #define BTPM_VF_REC 28
 // the facing test acosf(c) <= float(pi)/2 of the view-factor producer holds

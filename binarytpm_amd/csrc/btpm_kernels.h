@@ -111,8 +111,10 @@ extern "C" __global__ void btpm_status_kernel(const int* ids, const btpm_set_dev
 extern "C" __global__ void btpm_geom_facets(const double* equpos, const int* fv, int nf,
                                             int nv_primary, const double* trig,
                                             const double* frame, int s0, int nsteps, double* rec,
-                                            int* lit, float* cosang, float* sun, double sun_scale);
-extern "C" __global__ void btpm_geom_shadow(const double* rec, int nf, int nsteps, int* lit);
+                                            float4* flat, int* lit, float* cosang, float* sun,
+                                            double sun_scale);
+extern "C" __global__ void btpm_geom_shadow(const double* rec, const float4* flat, int nf,
+                                            int nsteps, int* lit);
 extern "C" __global__ void btpm_geom_finish(const int* lit, const float* cosang, const float* sun,
                                             int nf, int nsteps, int s0, int ntau, float solar,
                                             int* shadow, float* illum, float* sun_out);

@@ -26,21 +26,23 @@
 namespace {
 constexpr int kGR = BTPM_GEOM_REC;  // doubles per facet record
 // record layout: centroid[3], |centroid|, circumradius, centroid . normal,
-// normal[3], vertices[3][3], index (as double), pad
-constexpr int kMid = 0, kDist = 3, kRad = 4, kTc1 = 5, kNrm = 6, kVtx = 9, kIdx = 18;
-constexpr int kShChunk = 64;        // nearer-facet records staged per LDS chunk
+// normal[3], vertices[3][3]
+constexpr int kMid = 0, kDist = 3, kRad = 4, kTc1 = 5, kNrm = 6, kVtx = 9;
 }  // namespace
 
 // One (step, facet) per lane: the facet record of the step's chunk slot, the
 // back-face flag, cos(angle) and the unit Sun direction in the facet frame.
 //   trig[s] = (cos, sin) of the primary's and the secondary's rotation angle
 //   frame[0..8] = ecliptic <- equatorial matrix (row-major), frame[9..11] =
-//   heliocentric position of the system (km)
+//   heliocentric position of the system (km), frame[12..17] = two unit vectors
+//   across the direction to it, frame[18] = slack of the shadow tests' cull
+// flat[s][f] = the centroid seen along that direction, relative to the system's
+// position, and the square of the cull's reach (float, see btpm_geom_shadow)
 extern "C" __global__ __launch_bounds__(256) void btpm_geom_facets(
     const double* __restrict__ equpos, const int* __restrict__ fv, int nf, int nv_primary,
     const double* __restrict__ trig, const double* __restrict__ frame, int s0, int nsteps,
-    double* __restrict__ rec, int* __restrict__ lit, float* __restrict__ cosang,
-    float* __restrict__ sun, double sun_scale) {
+    double* __restrict__ rec, float4* __restrict__ flat, int* __restrict__ lit,
+    float* __restrict__ cosang, float* __restrict__ sun, double sun_scale) {
   const int f = blockIdx.x * blockDim.x + threadIdx.x;
   const int sl = blockIdx.y;
   if (f >= nf || sl >= nsteps) return;
@@ -116,8 +118,11 @@ extern "C" __global__ __launch_bounds__(256) void btpm_geom_facets(
   r[kDist] = t;
   r[kRad] = sqrt(r2);
   r[kTc1] = (mid[0] * n[0]) + (mid[1] * n[1]) + (mid[2] * n[2]);
-  r[kIdx] = (double)f;
-  r[kIdx + 1] = 0.0;
+  const double w0 = mid[0] - frame[9], w1 = mid[1] - frame[10], w2 = mid[2] - frame[11];
+  const float reach = (float)(sqrt(r2) + frame[18]);
+  flat[o] = make_float4((float)(w0 * frame[12] + w1 * frame[13] + w2 * frame[14]),
+                        (float)(w0 * frame[15] + w1 * frame[16] + w2 * frame[17]),
+                        reach * reach * 1.00001f, 0.0f);
 }
 
 namespace {
@@ -151,66 +156,86 @@ __device__ __forceinline__ bool ray_hits(const double (&g)[3], const double* __r
 }
 }  // namespace
 
-// Shadow flags of one step: a workgroup owns 256 facets G of a step (lane =
-// G) and walks every facet H of the step in LDS chunks of 64 records.  H is
-// tested against G if it is nearer the Sun (|H| < |G|, ties to the lower
-// index: the pair order of thermal.cpp:1686-1701), and only if the Sun->G
-// ray passes within H's circumradius + margin of H's centroid, measured in
-// the body's frame (w = H - G, |w|^2 - (w.u)^2 with u the unit ray): the
-// rounding of that distance and of the plane intersection is ~1e-16 |G|
-// (1e-8 km at 1 AU), the margin 1e-6 km + 1e-14 |G|, so a skipped H is one
-// whose triangle the ray misses by far more than the edge tests can resolve,
-// and the flags equal testing every pair.
-extern "C" __global__ __launch_bounds__(256) void btpm_geom_shadow(const double* __restrict__ rec,
-                                                                   int nf, int nsteps,
-                                                                   int* __restrict__ lit) {
-  __shared__ double H[kShChunk][kGR];
-  const int tid = (int)threadIdx.x;
-  const int f = blockIdx.x * blockDim.x + tid;
+// Shadow flags of one step, one wave per 64 facets G (lane = G).  H is tested
+// against G if it is nearer the Sun (|H| < |G|, ties to the lower index: the
+// pair order of thermal.cpp:1686-1701), and only if the Sun->G ray passes
+// within H's circumradius + margin of H's centroid, measured in the body's
+// frame (w = H - G, |w|^2 - (w.u)^2 with u the unit ray): the rounding of that
+// distance and of the plane intersection is ~1e-16 |G| (1e-8 km at 1 AU), the
+// margin 1e-6 km + 1e-14 |G|, so a skipped H is one whose triangle the ray
+// misses by far more than the edge tests can resolve, and the flags equal
+// testing every pair.
+//
+// Almost every pair is skipped, so which ones is settled in two dimensions and
+// 32 bits first: seen along the direction to the system the rays are points
+// (flat), their true directions turned by at most B/D of it (B the farthest
+// vertex from the system's position, D its distance).  The cull's reach adds
+// to the circumradius the margin, the 2 B^2/D by which a turned ray can pass
+// closer, four times over, and 4e-6 B for the 32-bit roundings; with B > D/2
+// it is infinite and nothing is culled.  A wave takes 64 H at a time, a lane
+// each, against the box around its own facets (neighbours in a mesh are near
+// each other), then the H that are left one by one against its facets, and
+// only the pairs left then in 64 bits.  1600 facets x 1950 steps, bound by
+// vector issue: every pair in 64 bits 2.20 ms, this 0.48 ms.
+extern "C" __global__ __launch_bounds__(256) void btpm_geom_shadow(
+    const double* __restrict__ rec, const float4* __restrict__ flat, int nf, int nsteps,
+    int* __restrict__ lit) {
+  const int lane = (int)threadIdx.x & 63;
+  const int f = blockIdx.x * blockDim.x + (int)threadIdx.x;
   const int sl = blockIdx.y;
   if (sl >= nsteps) return;  // uniform
   const double* R = rec + (size_t)sl * nf * kGR;
+  const float4* P = flat + (size_t)sl * nf;
   const bool in = f < nf;
-  int on = 0;
-  double g[3] = {0.0, 0.0, 0.0}, u[3] = {0.0, 0.0, 0.0}, gd = 0.0;
-  if (in) {
-    on = lit[(size_t)sl * nf + f];
-    const double* G = R + (size_t)f * kGR;
-    g[0] = G[kMid];
-    g[1] = G[kMid + 1];
-    g[2] = G[kMid + 2];
-    gd = G[kDist];
-    u[0] = g[0] / gd;
-    u[1] = g[1] / gd;
-    u[2] = g[2] / gd;
-  }
-  if (__syncthreads_count(on) == 0) return;
+  const int was = in ? lit[(size_t)sl * nf + f] : 0;
+  int on = was;
+  if (__ballot(on) == 0) return;
+  const double* G = R + (size_t)(in ? f : nf - 1) * kGR;
+  const double g[3] = {G[kMid], G[kMid + 1], G[kMid + 2]};
+  const double gd = G[kDist];
+  const double u[3] = {g[0] / gd, g[1] / gd, g[2] / gd};
   // skip margin: well above the ~1e-16 |G| rounding of w and of the plane
   // intersection, well below any facet
   const double margin = 1e-6 + 1e-14 * gd;
-  for (int c0 = 0; c0 < nf; c0 += kShChunk) {
-    const int nc = min(kShChunk, nf - c0);
-    __syncthreads();
-    for (int e = tid; e < nc * kGR; e += (int)blockDim.x)
-      (&H[0][0])[e] = R[(size_t)c0 * kGR + e];
-    __syncthreads();
-    if (!on) continue;
-    for (int h = 0; h < nc; ++h) {
-      const double hd = H[h][kDist];
-      const int hi = c0 + h;
-      if (!(hd < gd || (hd == gd && hi < f))) continue;
-      const double w0 = H[h][kMid] - g[0], w1 = H[h][kMid + 1] - g[1], w2 = H[h][kMid + 2] - g[2];
+  const float4 p = P[in ? f : nf - 1];
+  const float inf = __builtin_inff();
+  float x0 = on ? p.x : inf, x1 = on ? p.x : -inf, y0 = on ? p.y : inf, y1 = on ? p.y : -inf;
+  for (int o = 32; o > 0; o >>= 1) {
+    x0 = fminf(x0, __shfl_xor(x0, o));
+    x1 = fmaxf(x1, __shfl_xor(x1, o));
+    y0 = fminf(y0, __shfl_xor(y0, o));
+    y1 = fmaxf(y1, __shfl_xor(y1, o));
+  }
+  float4 next = P[min(lane, nf - 1)];
+  for (int c0 = 0; c0 < nf; c0 += 64) {
+    const float4 q = next;
+    next = P[min(c0 + 64 + lane, nf - 1)];
+    // a cull has to be certain: NaN compares false and culls nothing
+    const float bx = fmaxf(fmaxf(x0 - q.x, q.x - x1), 0.0f);
+    const float by = fmaxf(fmaxf(y0 - q.y, q.y - y1), 0.0f);
+    unsigned long long left = __ballot(c0 + lane < nf && !(bx * bx + by * by > q.z));
+    while (left != 0) {
+      const int l = __builtin_ctzll(left);
+      left &= left - 1;
+      const float dx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(q.x), l)) - p.x;
+      const float dy = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(q.y), l)) - p.y;
+      const float r2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(q.z), l));
+      const bool close = on && !(dx * dx + dy * dy > r2);
+      if (__ballot(close) == 0) continue;
+      const int hi = c0 + l;
+      const double* H = R + (size_t)hi * kGR;
+      const double hd = H[kDist];
+      if (!(close && (hd < gd || (hd == gd && hi < f)))) continue;
+      const double w0 = H[kMid] - g[0], w1 = H[kMid + 1] - g[1], w2 = H[kMid + 2] - g[2];
       const double wu = w0 * u[0] + w1 * u[1] + w2 * u[2];
       const double d2 = (w0 * w0 + w1 * w1 + w2 * w2) - wu * wu;
-      const double reach = H[h][kRad] + margin;
+      const double reach = H[kRad] + margin;
       if (d2 > reach * reach) continue;
-      if (ray_hits(g, H[h])) {
-        on = 0;
-        break;
-      }
+      if (ray_hits(g, H)) on = 0;
     }
+    if (__ballot(on) == 0) break;
   }
-  if (in) lit[(size_t)sl * nf + f] = on;
+  if (on != was) lit[(size_t)sl * nf + f] = on;
 }
 
 // [step][facet] staging of a chunk -> [facet][step] outputs, through a
@@ -278,7 +303,7 @@ extern "C" int btpm_geometry_illumination(btpm_ctx* ctx, const btpm_geometry* g,
   const int nv = g->nv, nf = g->nf, ntau = g->ntau;
   // the reference's trigonometry, on the host (thermal.cpp:12, 1274-1296, 1349, 1371)
   const double PI = 4.0 * std::atan(1.0);
-  double frame[12];
+  double frame[19];
   {
     const double r0 = g->rot[0], r1 = g->rot[1];
     const double gamma = std::acos(std::cos(r0) * std::sin(std::fabs(r1)));
@@ -297,6 +322,37 @@ extern "C" int btpm_geometry_illumination(btpm_ctx* ctx, const btpm_geometry* g,
     frame[10] = g->au_km * g->pol[0] * std::cos(g->pol[1]) * std::sin(g->pol[2]);
     frame[11] = g->au_km * g->pol[0] * std::sin(g->pol[1]);
   }
+  {
+    // two unit vectors across the direction to the system, and the cull's slack
+    double d = 0.0, far2 = 0.0;
+    for (int k = 0; k < 3; ++k) d += frame[9 + k] * frame[9 + k];
+    d = std::sqrt(d);
+    for (int v = 0; v < g->nv; ++v) {
+      const double* e = g->equpos + 3 * (size_t)v;
+      const double r2 = e[0] * e[0] + e[1] * e[1] + e[2] * e[2];
+      if (r2 > far2) far2 = r2;  // a facet with a NaN casts and takes no shadow
+    }
+    const double n[3] = {frame[9] / d, frame[10] / d, frame[11] / d};
+    int m = 0;  // the axis farthest from the direction
+    for (int k = 1; k < 3; ++k)
+      if (std::fabs(n[k]) < std::fabs(n[m])) m = k;
+    double* e1 = frame + 12;
+    double* e2 = frame + 15;
+    double l = 0.0;
+    for (int k = 0; k < 3; ++k) {
+      e1[k] = (k == m ? 1.0 : 0.0) - n[m] * n[k];
+      l += e1[k] * e1[k];
+    }
+    for (int k = 0; k < 3; ++k) e1[k] /= std::sqrt(l);
+    for (int k = 0; k < 3; ++k)
+      e2[k] = n[(k + 1) % 3] * e1[(k + 2) % 3] - n[(k + 2) % 3] * e1[(k + 1) % 3];
+    double norm2 = 0.0;  // the matrix is a rotation only up to the pole's formula
+    for (int k = 0; k < 9; ++k) norm2 += frame[k] * frame[k];
+    const double far = std::sqrt(far2 * norm2);
+    frame[18] = far <= 0.5 * d
+                    ? 8.0 * far * far / d + 4e-6 * far + 2e-6 + 2e-14 * (d + far)
+                    : INFINITY;
+  }
   const float sol = (float)(1367.0 / (g->pol[0] * g->pol[0]));
   if (solar) *solar = sol;
   std::vector<double> trig(4 * (size_t)ntau);
@@ -312,7 +368,7 @@ extern "C" int btpm_geometry_illumination(btpm_ctx* ctx, const btpm_geometry* g,
   upload(d_eq, g->equpos, 3 * (size_t)nv, st);
   upload(d_fv, g->facets, 3 * (size_t)nf, st);
   upload(d_trig, trig.data(), trig.size(), st);
-  upload(d_frame, frame, 12, st);
+  upload(d_frame, frame, 19, st);
   const size_t nser = (size_t)nf * ntau;
   DBuf d_shadow, d_illum, d_sun;
   d_shadow.alloc(nser * sizeof(int));
@@ -322,7 +378,8 @@ extern "C" int btpm_geometry_illumination(btpm_ctx* ctx, const btpm_geometry* g,
   const size_t rec_step = (size_t)nf * BTPM_GEOM_REC * sizeof(double);
   const int sc = (int)std::max<size_t>(1, std::min<size_t>({(size_t)ntau, (256u << 20) / rec_step,
                                                              (size_t)65535}));
-  DBuf d_rec, d_lit, d_cos, d_sunc;
+  DBuf d_rec, d_flat, d_lit, d_cos, d_sunc;
+  d_flat.alloc((size_t)sc * nf * sizeof(float4));
   d_rec.alloc(rec_step * sc);
   d_lit.alloc((size_t)sc * nf * sizeof(int));
   d_cos.alloc((size_t)sc * nf * sizeof(float));
@@ -331,10 +388,10 @@ extern "C" int btpm_geometry_illumination(btpm_ctx* ctx, const btpm_geometry* g,
     const int ns = std::min(sc, ntau - s0);
     hipLaunchKernelGGL(btpm_geom_facets, dim3(grid1(nf, 256), ns), dim3(256), 0, st,
                        d_eq.as<double>(), d_fv.as<int>(), nf, g->nv_primary, d_trig.as<double>(),
-                       d_frame.as<double>(), s0, ns, d_rec.as<double>(), d_lit.as<int>(),
+                       d_frame.as<double>(), s0, ns, d_rec.as<double>(), d_flat.as<float4>(), d_lit.as<int>(),
                        d_cos.as<float>(), d_sunc.as<float>(), g->sun_scale);
     hipLaunchKernelGGL(btpm_geom_shadow, dim3(grid1(nf, 256), ns), dim3(256), 0, st,
-                       d_rec.as<double>(), nf, ns, d_lit.as<int>());
+                       d_rec.as<double>(), d_flat.as<float4>(), nf, ns, d_lit.as<int>());
     hipLaunchKernelGGL(btpm_geom_finish, dim3(grid1(nf, 64), grid1(ns, 64)), dim3(256), 0, st,
                        d_lit.as<int>(), d_cos.as<float>(), d_sunc.as<float>(), nf, ns, s0, ntau, sol,
                        d_shadow.as<int>(), d_illum.as<float>(),

@@ -110,3 +110,17 @@ def test_crater_sunlight_parity(ctx):
     mism = int((g[0] != o[0]).sum()) + int((g[1] != o[1]).sum())
     print(f"[parity] crater sunlight chain: {mism} mismatches of {2 * g[0].size}", flush=True)
     assert mism == 0
+
+
+@pytest.mark.parametrize("nf", [1, 63, 64, 65, 100, 200])
+@pytest.mark.parametrize("au_km", [149597870.7, 60.0, 4.0])
+def test_shadow_cull_edges(ctx, nf, au_km):
+    """Facets in no order, counts around a wave, and a Sun so near that the
+    rays are far from parallel (4 km: nothing may be culled)."""
+    equ, fv, npv = inputs.binary_shape(1, 1, sep=1.4, dent=0.35)
+    fv = np.random.default_rng(5).permutation(fv)[:nf]
+    kw = dict(nv_primary=npv, rev_primary=3.0, rev_secondary=1.0, au_km=au_km)
+    pos, pole = (1.0, 0.05, 0.3), (1.2, 0.7)
+    gpu = th.geometry_illumination(ctx, equ, fv, 70, pos, pole, **kw)
+    ref = O.geometry(equ, fv, 70, pos, pole, **kw)
+    assert np.array_equal(gpu.shadow, ref.shadow)

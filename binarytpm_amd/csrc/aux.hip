@@ -511,17 +511,32 @@ extern "C" __global__ __launch_bounds__(256) void btpm_pack_drf(const int* __res
 // sub-facet's sunlit fraction is interpolated bilinearly in vis_table
 // [n_el][n_az][100] (elevation i*90/(n_el-1) deg, azimuth i*360/n_az deg)
 // and its cosine is max(0, n_j . u) with the unit direction u.
-// rgi [f][s][j] may be null.  Output illum blocked [b][f*NS+j][k].  One
-// workgroup (128 lanes) per (facet, block): lane j holds the 8 steps of
-// sub-facet j.
+// rgi [f][s][j] may be null.  Output illum blocked [b][f*NS+j][k].
+//
+// One workgroup (4 waves) per facet and 32 steps.  A sweep is the product of
+// the 100 x 100 view factors with 32 columns on the FP32 matrix instructions
+// (16x16x4, the rate of two FMAs per lane): wave w owns the rows of tiles w and
+// w + 4, keeps their factors in registers for all sweeps (50 floats per lane)
+// and reads the columns from LDS, where each wave puts its own rows of the
+// next sweep.  A lane's four rows of a tile are the four K entries it needs as
+// an input, so both go as one 16-byte access.  The sweeps of a block of 8
+// steps end when none of its values moves by more than acc, as if it were
+// alone.  1280 facets x 650 steps: a dot product per lane and step, both
+// operands from LDS, 6.4 ms; this 0.90 ms.
 // ---------------------------------------------------------------------------
 namespace {
-__device__ __forceinline__ float direct_from_sun(const float* __restrict__ d3,
-                                                 const float* __restrict__ vis, int n_el,
-                                                 int n_az, float nx, float ny, float nz, int j) {
+constexpr int kScCols = 32;               // steps per workgroup
+constexpr int kScBlk = kScCols / BTPM_BLK;
+typedef float fvec4 __attribute__((ext_vector_type(4)));
+struct SunCell {  // where a Sun direction falls in the table
+  float len, ux, uy, uz, we, wa;
+  int i00, i01, i10, i11;
+};
+__device__ __forceinline__ SunCell sun_cell(const float* __restrict__ d3, int n_el, int n_az) {
+  SunCell c{};
   const float dx = d3[0], dy = d3[1], dz = d3[2];
   const float len = sqrtf(dx * dx + dy * dy + dz * dz);
-  if (!(len > 0.0f) || !(dz > 0.0f)) return 0.0f;
+  if (!(len > 0.0f) || !(dz > 0.0f)) return c;  // len 0: no light
   const float il = 1.0f / len;
   const double ux = (double)(dx * il), uy = (double)(dy * il), uz = (double)(dz * il);
   const double kPi = 3.14159265358979323846;
@@ -532,99 +547,191 @@ __device__ __forceinline__ float direct_from_sun(const float* __restrict__ d3,
   const double fa = az / (2.0 * kPi / n_az);
   const int ie = (int)floor(fe);
   const int ia = ((int)floor(fa)) % n_az;
-  const float we = (float)(fe - ie), wa = (float)(fa - floor(fa));
   const int ie1 = min(ie + 1, n_el - 1), ia1 = (ia + 1) % n_az;
-  const float v00 = vis[((size_t)ie * n_az + ia) * BTPM_NS + j];
-  const float v01 = vis[((size_t)ie * n_az + ia1) * BTPM_NS + j];
-  const float v10 = vis[((size_t)ie1 * n_az + ia) * BTPM_NS + j];
-  const float v11 = vis[((size_t)ie1 * n_az + ia1) * BTPM_NS + j];
-  const float v = (1.0f - we) * ((1.0f - wa) * v00 + wa * v01) +
-                  we * ((1.0f - wa) * v10 + wa * v11);
-  const float c = (float)ux * nx + (float)uy * ny + (float)uz * nz;
-  return (v * len) * (c > 0.0f ? c : 0.0f);
+  c.len = len;
+  c.ux = (float)ux;
+  c.uy = (float)uy;
+  c.uz = (float)uz;
+  c.we = (float)(fe - ie);
+  c.wa = (float)(fa - floor(fa));
+  c.i00 = ie * n_az + ia;
+  c.i01 = ie * n_az + ia1;
+  c.i10 = ie1 * n_az + ia;
+  c.i11 = ie1 * n_az + ia1;
+  return c;
+}
+__device__ __forceinline__ float sun_direct(const SunCell& c, const float* __restrict__ vis,
+                                            const float* __restrict__ n, int j) {
+  if (!(c.len > 0.0f)) return 0.0f;
+  auto at = [&](int i) { return vis[(size_t)i * BTPM_NS + j]; };
+  const float v = (1.0f - c.we) * ((1.0f - c.wa) * at(c.i00) + c.wa * at(c.i01)) +
+                  c.we * ((1.0f - c.wa) * at(c.i10) + c.wa * at(c.i11));
+  const float d = c.ux * n[0] + c.uy * n[1] + c.uz * n[2];
+  return (v * c.len) * (d > 0.0f ? d : 0.0f);
 }
 }  // namespace
 
-extern "C" __global__ __launch_bounds__(128) void btpm_crater_scatter(
+extern "C" __global__ __launch_bounds__(256) void btpm_crater_scatter(
     const float* __restrict__ vf32, const float* __restrict__ albedo,
     const float* __restrict__ shadow, const float* __restrict__ cosang,
     const float* __restrict__ sun, const float* __restrict__ vis_table, int n_el, int n_az,
     const float* __restrict__ normals, const float* __restrict__ rgi, float solar, int multiple,
     float acc, int max_iter, int nfac, int ntau, int nb, float* __restrict__ illum_out) {
-  __shared__ float vfs[BTPM_NS * BTPM_NS];
-  __shared__ float il[BTPM_BLK][BTPM_NS];
+  constexpr int NS = BTPM_NS;
+  __shared__ __align__(16) float il[2][kScCols * NS];  // [column][row]
+  __shared__ SunCell cell[kScCols];
+  __shared__ int moved[3];
   const int f = blockIdx.y;
-  const int b = blockIdx.x;
-  const int j = threadIdx.x;
-  const bool ok = j < BTPM_NS;
-  for (int e = j; e < BTPM_NS * BTPM_NS; e += 128) vfs[e] = vf32[e];
-  const float a = albedo[f];
-  float nx = 0.0f, ny = 0.0f, nz = 0.0f;
-  if (sun && ok) {
-    nx = normals[3 * j];
-    ny = normals[3 * j + 1];
-    nz = normals[3 * j + 2];
-  }
-  float sp[BTPM_BLK], res[BTPM_BLK];
-#pragma unroll
-  for (int k = 0; k < BTPM_BLK; ++k) {
-    const int s = min(b * BTPM_BLK + k, ntau - 1);
-    sp[k] = 0.0f;
-    if (ok) {
-      const size_t o = ((size_t)f * ntau + s) * BTPM_NS + j;
-      const float direct =
-          sun ? direct_from_sun(sun + ((size_t)f * ntau + s) * 3, vis_table, n_el, n_az, nx, ny,
-                                nz, j)
-              : shadow[o] * cosang[o];
-      sp[k] = solar * direct + (rgi ? rgi[o] : 0.0f);
-      il[k][j] = sp[k];
-    }
-  }
-  __syncthreads();
-  // single scattering: tot_j = il_j + A sum_i VF(j->i) il_i, clamped >= 0
-#pragma unroll
-  for (int k = 0; k < BTPM_BLK; ++k) {
-    float t = sp[k];
-    if (ok)
-      for (int i = 0; i < BTPM_NS; ++i) t = fmaf(vfs[i * BTPM_NS + j] * a, il[k][i], t);
-    res[k] = t > 0.0f ? t : 0.0f;
-  }
-  if (multiple && a > 0.0f) {
-    // Jacobi on p = A (sp + VF p) from p = A * single; stop when every
-    // |p_new - p_old| <= acc over the block's 8 steps
+  const int s0 = blockIdx.x * kScCols;
+  const int tid = (int)threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int g4 = 4 * (lane >> 4), n = lane & 15;
+  if (tid < 3) moved[tid] = 0;
+  if (sun) {
+    if (tid < kScCols)
+      cell[tid] = sun_cell(sun + ((size_t)f * ntau + min(s0 + tid, ntau - 1)) * 3, n_el, n_az);
     __syncthreads();
+  }
+  const float a = albedo[f];
+  // the factors: row 16 t + n, entry q of K group kk is 16 kk + g4 + q, the
+  // last four entries one per lane group
+  float vf[2][25];
 #pragma unroll
-    for (int k = 0; k < BTPM_BLK; ++k)
-      if (ok) il[k][j] = a * res[k];
-    for (int it = 0; it < max_iter; ++it) {
-      __syncthreads();  // the a*res / previous sweep writes are visible
-      float pn[BTPM_BLK];
-      int ch = 0;
+  for (int m = 0; m < 2; ++m) {
+    const int row = 16 * (wave + 4 * m) + n;
 #pragma unroll
-      for (int k = 0; k < BTPM_BLK; ++k) {
-        float sum = 0.0f;
-        if (ok)
-          for (int i = 0; i < BTPM_NS; ++i) sum = fmaf(vfs[i * BTPM_NS + j], il[k][i], sum);
-        pn[k] = a * (sp[k] + sum);
-        if (ok && fabsf(pn[k] - il[k][j]) > acc) ch = 1;
-      }
-      __syncthreads();  // every lane has read the old sweep
-#pragma unroll
-      for (int k = 0; k < BTPM_BLK; ++k)
-        if (ok) il[k][j] = pn[k];
-      if (!__syncthreads_or(ch)) break;  // block-uniform exit
+    for (int k = 0; k < 25; ++k) {
+      const int i = k < 24 ? 16 * (k / 4) + g4 + k % 4 : 96 + (lane >> 4);
+      vf[m][k] = row < NS ? vf32[i * NS + row] : 0.0f;
     }
+  }
+  // this lane's rows j0(m) .. j0(m) + 3 of columns n and 16 + n
+  const int j0[2] = {16 * wave + g4, 16 * (wave + 4) + g4};
+  const bool ok[2] = {true, j0[1] < NS};
+  fvec4 sp[2][2], own[2][2];
 #pragma unroll
-    for (int k = 0; k < BTPM_BLK; ++k) res[k] = ok ? il[k][j] / a : 0.0f;
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      sp[m][t] = fvec4{0.0f, 0.0f, 0.0f, 0.0f};
+      if (!ok[m]) continue;
+      const int col = 16 * t + n;
+      const size_t o = ((size_t)f * ntau + min(s0 + col, ntau - 1)) * NS + j0[m];
+      fvec4 direct;
+      if (sun) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          direct[r] = sun_direct(cell[col], vis_table, normals + 3 * (j0[m] + r), j0[m] + r);
+      } else {
+        direct = *reinterpret_cast<const fvec4*>(shadow + o) *
+                 *reinterpret_cast<const fvec4*>(cosang + o);
+      }
+      fvec4 x = {0.0f, 0.0f, 0.0f, 0.0f};
+      if (rgi) x = *reinterpret_cast<const fvec4*>(rgi + o);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x[r] = fmaf(solar, direct[r], x[r]);
+      sp[m][t] = x;
+      *reinterpret_cast<fvec4*>(&il[0][col * NS + j0[m]]) = x;
+    }
+  __syncthreads();
+  // sum[j] = sum_i VF(j->i) il[i] of the columns in a buffer
+  auto sweep = [&](const float* b, fvec4 (&sum)[2][2]) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const float* x = b + (16 * t + n) * NS;
+      sum[0][t] = sum[1][t] = fvec4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int kk = 0; kk < 6; ++kk) {
+        const fvec4 e = *reinterpret_cast<const fvec4*>(x + 16 * kk + g4);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int m = 0; m < 2; ++m)
+            if (m == 0 || wave < 3)
+              sum[m][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[m][4 * kk + q], e[q], sum[m][t],
+                                                               0, 0, 0);
+      }
+      const float e = x[96 + (lane >> 4)];
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+        if (m == 0 || wave < 3)
+          sum[m][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[m][24], e, sum[m][t], 0, 0, 0);
+    }
+  };
+  auto put = [&](float* b, float scale) {
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        if (ok[m]) *reinterpret_cast<fvec4*>(&b[(16 * t + n) * NS + j0[m]]) = scale * own[m][t];
+  };
+  fvec4 sum[2][2];
+  int cur = 0;
+  // single scattering: tot_j = il_j + A sum_i VF(j->i) il_i, clamped >= 0
+  sweep(il[0], sum);
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float v = fmaf(a, sum[m][t][r], sp[m][t][r]);
+        own[m][t][r] = v > 0.0f ? v : 0.0f;
+      }
+  if (multiple && a > 0.0f) {
+    // Jacobi on p = A (sp + VF p) from p = A * single; a block of 8 steps
+    // stops when every |p_new - p_old| <= acc in it.  own holds p / A, the
+    // result, so that it is not multiplied by A and divided again
+    cur = 1;
+    put(il[1], a);
+    __syncthreads();
+    int run = (1 << kScBlk) - 1;  // blocks still moving
+    for (int it = 0; it < max_iter; ++it) {
+      sweep(il[cur], sum);
+      int mine = 0;
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const int bit = 1 << (2 * t + (n >> 3));
+        bool ch = false;
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float x = sp[m][t][r] + sum[m][t][r];
+            ch |= ok[m] && fabsf(a * x - a * own[m][t][r]) > acc;
+            own[m][t][r] = (run & bit) ? x : own[m][t][r];
+          }
+        const unsigned long long c = __ballot(ch);
+        mine |= (c & 0x00ff00ff00ff00ffull ? 1 << (2 * t) : 0) |
+                (c & 0xff00ff00ff00ff00ull ? 2 << (2 * t) : 0);
+      }
+      if (lane == 0 && mine != 0) atomicOr(&moved[it % 3], mine);
+      put(il[cur ^ 1], a);
+      __syncthreads();
+      cur ^= 1;
+      run &= moved[it % 3];
+      // free for the sweep after next: every wave has read it
+      if (tid == 0) moved[(it + 2) % 3] = 0;
+      if (run == 0) break;  // the same for every wave
+    }
   } else if (multiple) {
 #pragma unroll
-    for (int k = 0; k < BTPM_BLK; ++k) res[k] = sp[k];
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) own[m][t] = sp[m][t];
   }
-  if (!ok) return;
-  const int ncols = nfac * BTPM_NS;
-  float4* o = reinterpret_cast<float4*>(illum_out + ((size_t)b * ncols + f * BTPM_NS + j) * BTPM_BLK);
-  o[0] = make_float4(res[0], res[1], res[2], res[3]);
-  o[1] = make_float4(res[4], res[5], res[6], res[7]);
+  // out through the buffer that the last sweep did not read
+  put(il[cur ^ 1], 1.0f);
+  __syncthreads();
+  const int ncols = nfac * NS;
+  for (int e = tid; e < kScBlk * NS; e += 256) {
+    const int bl = e / NS, j = e - bl * NS, b = s0 / BTPM_BLK + bl;
+    if (b >= nb) break;
+    const float* x = &il[cur ^ 1][bl * BTPM_BLK * NS + j];
+    float4* o = reinterpret_cast<float4*>(illum_out + ((size_t)b * ncols + f * NS + j) * BTPM_BLK);
+    o[0] = make_float4(x[0], x[NS], x[2 * NS], x[3 * NS]);
+    o[1] = make_float4(x[4 * NS], x[5 * NS], x[6 * NS], x[7 * NS]);
+  }
 }
 
 // ---------------------------------------------------------------------------

@@ -567,7 +567,7 @@ void GPU_sfcpartialshadow(int* shadow_H, float* sfc_shadow_H, float* sfc_illumve
 static void scatter(float solar, int multiple, float acc) {
   Compat& c = C();
   if (!c.illum.p) c.illum.alloc(blk() * 4);
-  hipLaunchKernelGGL(btpm_crater_scatter, dim3(c.nb, c.nf), dim3(128), 0, c.ctx->stream,
+  hipLaunchKernelGGL(btpm_crater_scatter, dim3((c.nb + 3) / 4, c.nf), dim3(256), 0, c.ctx->stream,
                      c.vf32.as<float>(), c.albedo.as<float>(), c.sfc_shadow.as<float>(),
                      c.illumangle.as<float>(), (const float*)nullptr, (const float*)nullptr, 0, 0,
                      (const float*)nullptr, c.rgi.as<float>(), solar, multiple, acc, 100000,

@@ -1997,7 +1997,7 @@ int btpm_shape_create(btpm_ctx* ctx, const btpm_params* p, const btpm_body* body
         rgip = rgi.as<float>();
       }
       const float acc = crater->scatter_acc > 0 ? crater->scatter_acc : 1e-4f;
-      hipLaunchKernelGGL(btpm_crater_scatter, dim3(nb, nf), dim3(128), 0, st,
+      hipLaunchKernelGGL(btpm_crater_scatter, dim3((nb + 3) / 4, nf), dim3(256), 0, st,
                          sh->cvf32.as<float>(), sh->albedo.as<float>(), dsh.as<float>(),
                          dcos.as<float>(), dsun.as<float>(), dvis.as<float>(),
                          by_sun ? crater->n_el : 0, by_sun ? crater->n_az : 0, dnrm.as<float>(),

@@ -905,17 +905,28 @@ extern "C" __global__ __launch_bounds__(kSHRows) void btpm_selfheat_tiled(
 // prefetched; each lane still adds its entries in emitter order, so the sums
 // equal btpm_selfheat_tiled's bit for bit.  The next chunk's emission rows
 // are fetched into registers while the current chunk is consumed.
+//
+// The LDS reads bound it: 4 bytes per multiply-add from 64 rows that have
+// nothing to do with each other.  A row is a whole number of sweeps over the
+// banks and lane l takes its 16-byte pieces in the order l ^ q, so lanes served
+// together read different pieces whatever their rows (all lanes on the same
+// piece of rows padded to H + 4 floats: two to three lanes on a bank).  H = 64
+// then meets no conflict; two rows of 32 can still share half the banks, but
+// H = 32 holds twice the waves.  5120 x 154 factors, 650 steps, 8 sets in one
+// launch: H = 64 646 us before, 567 now; H = 32 573 before, 545 now.  512
+// receivers per workgroup with H = 64 (no rows ahead in registers, 16 waves
+// per CU) take 543 for 8 sets but 254 against 234 for 4 and 220 against 70 for
+// one.
 template <int H>
 __device__ __forceinline__ void selfheat_ell_body(const int2* __restrict__ wseg,
                                                   const int2* __restrict__ ent, int nf,
                                                   int nchunk, const int* __restrict__ slots,
                                                   const btpm_set_dev* __restrict__ sets,
                                                   const btpm_status_dev* __restrict__ status) {
-  constexpr int kStride = H + 4;                     // LDS row stride in floats
   constexpr int kQ4 = H / 4;                         // float4 per emission row
   constexpr int kPer = kSHChunk * kQ4 / kSHRows;     // float4 staged per lane
   static_assert(kSHChunk * kQ4 % kSHRows == 0 && kSHRows % kQ4 == 0, "staging shape");
-  __shared__ __align__(16) float E[kSHChunk * kStride];
+  __shared__ __align__(16) float E[kSHChunk * H];
   const int slot = slots[blockIdx.z];
   if (status[slot].done) return;
   const btpm_set_dev& S = sets[slot];
@@ -943,9 +954,11 @@ __device__ __forceinline__ void selfheat_ell_body(const int2* __restrict__ wseg,
       if (g < nf && scol) pre[i] = gload4(emis + (size_t)g * npad + s0 + sq4);
     }
   };
-  float acc[H];
+  // acc[q]: steps 4 ((lane ^ q) % kQ4) .. + 3
+  float4 acc[kQ4];
 #pragma unroll
-  for (int q = 0; q < H; ++q) acc[q] = 0.0f;
+  for (int q = 0; q < kQ4; ++q) acc[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  const unsigned turn = 16u * (lane & (kQ4 - 1));  // in bytes
   // the wave's segment (first, n) of a chunk is wave-uniform; read through
   // an opaque zero VGPR it comes by a vector load, one chunk ahead (a scalar
   // load would share the LDS wait counter, and the chunk's first LDS wait
@@ -959,7 +972,7 @@ __device__ __forceinline__ void selfheat_ell_body(const int2* __restrict__ wseg,
     __syncthreads();  // the previous chunk has been consumed
 #pragma unroll
     for (int i = 0; i < kPer; ++i)
-      *reinterpret_cast<float4*>(&E[(srow + i * (kSHRows / kQ4)) * kStride + sq4]) = pre[i];
+      *reinterpret_cast<float4*>(&E[(srow + i * (kSHRows / kQ4)) * H + sq4]) = pre[i];
     if (c + 1 < nchunk) fetch(c + 1);
     const int2 dc = dn;
     dn = wsb[(size_t)min(c + 1, nchunk - 1) * BTPM_SH_WAVES + vz];
@@ -978,14 +991,15 @@ __device__ __forceinline__ void selfheat_ell_body(const int2* __restrict__ wseg,
       int gx = gv.x;
       asm volatile("" : "+v"(gx));
       const float v = __int_as_float(gv.y);
-      const float* er = &E[gx * kStride];
+      // one instruction per address: byte offsets, the piece by exclusive or
+      const unsigned er = (unsigned)gx * (4u * H) | turn;
 #pragma unroll
-      for (int q = 0; q < H; q += 4) {
-        const float4 e4 = *reinterpret_cast<const float4*>(er + q);
-        acc[q] = fmaf(v, e4.x, acc[q]);
-        acc[q + 1] = fmaf(v, e4.y, acc[q + 1]);
-        acc[q + 2] = fmaf(v, e4.z, acc[q + 2]);
-        acc[q + 3] = fmaf(v, e4.w, acc[q + 3]);
+      for (int q = 0; q < kQ4; ++q) {
+        const float4 e4 = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(E) + (er ^ (16u * q)));
+        acc[q].x = fmaf(v, e4.x, acc[q].x);
+        acc[q].y = fmaf(v, e4.y, acc[q].y);
+        acc[q].z = fmaf(v, e4.z, acc[q].z);
+        acc[q].w = fmaf(v, e4.w, acc[q].w);
       }
     };
     int2 qa = e[0], qb = e[(size_t)min(1, last) * 64], qc = e[(size_t)min(2, last) * 64];
@@ -1008,17 +1022,18 @@ __device__ __forceinline__ void selfheat_ell_body(const int2* __restrict__ wseg,
   if (!live) return;
   const float* __restrict__ src = S.src;
   float* __restrict__ y = S.qext;
+  // pieces 2m, 2m + 1 of a lane are the two halves of one block of 8 steps
 #pragma unroll
-  for (int bq = 0; bq < H / BTPM_BLK; ++bq) {
-    if (s0 + bq * BTPM_BLK >= npad) break;
-    const size_t o = ((size_t)(s0 / BTPM_BLK + bq) * nf + f) * BTPM_BLK;
+  for (int m = 0; m < kQ4 / 2; ++m) {
+    const int st = s0 + BTPM_BLK * (m ^ ((lane & (kQ4 - 1)) >> 1));
+    if (st >= npad) continue;
+    const float4 p = acc[2 * m], q = acc[2 * m + 1];
+    const float4 lo = lane & 1 ? q : p, hi = lane & 1 ? p : q;
+    const size_t o = ((size_t)(st / BTPM_BLK) * nf + f) * BTPM_BLK;
     const float4 a = gload4(src + o);
     const float4 b = gload4(src + o + 4);
-    const int q = bq * BTPM_BLK;
-    gstore4(y + o,
-            make_float4(a.x + acc[q], a.y + acc[q + 1], a.z + acc[q + 2], a.w + acc[q + 3]));
-    gstore4(y + o + 4,
-            make_float4(b.x + acc[q + 4], b.y + acc[q + 5], b.z + acc[q + 6], b.w + acc[q + 7]));
+    gstore4(y + o, make_float4(a.x + lo.x, a.y + lo.y, a.z + lo.z, a.w + lo.w));
+    gstore4(y + o + 4, make_float4(b.x + hi.x, b.y + hi.y, b.z + hi.z, b.w + hi.w));
   }
 }
 

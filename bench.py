@@ -879,7 +879,7 @@ def main():
             "latency_p50_s": float(np.percentile(lat, 50)),
             "latency_p99_s": float(np.percentile(lat, 99)),
             "roofline": {
-                "kernel": "btpm_conduct_crater",
+                "kernel": "btpm_conduct_crater_lin",
                 "bound": "hbm",
                 "achieved": achieved,
                 "peak": HBM_PEAK_GBS,
@@ -894,11 +894,12 @@ def main():
                 "bytes_per_column_step": BYTES_PER_COLSTEP,
                 "smooth_kernel_gbs": BYTES_PER_COLSTEP * sk_cs / sk_s / 1e9 if sk_s > 0 else 0.0,
                 "smooth_avg_launch_ms": 1000.0 * sk_s / max(sk_n, 1),
-                # the kernel's actual bound: VALU issue (SQ counters, committed summary)
+                # the kernel's VALU issue (SQ counters, committed summary)
                 "valu_instr_per_column_step": summary_value(VALU_FILE,
                                                             "valu_instr_per_column_step"),
                 "valu_issue_frac": summary_value(VALU_FILE, "valu_issue_frac"),
-                # the crater contraction on the matrix cores (executed FLOP incl. split)
+                # crater contraction and conduction operator on the matrix cores
+                # (executed FLOP incl. split)
                 "mfma_crater_product_tflops": (
                     summary_value(VALU_FILE, "mfma_flop_per_column_step") * ck_cs / ck_s / 1e12
                     if (ck_s > 0 and summary_value(VALU_FILE, "mfma_flop_per_column_step"))

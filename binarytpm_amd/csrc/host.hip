@@ -1490,14 +1490,14 @@ size_t stage_slice(size_t bytes) {
   return std::min(kStageSlice, std::max(kStageSliceMin, quarter));
 }
 
-// pinned host memory goes by DMA alone
-bool host_pinned(const void* p) {
-  hipPointerAttribute_t a;
+// memory that HIP knows (pinned, managed, device) goes by DMA alone
+bool dma_ready(const void* p) {
+  hipPointerAttribute_t a = {};
   if (hipPointerGetAttributes(&a, p) != hipSuccess) {
     (void)hipGetLastError();
     return false;
   }
-  return a.type == hipMemoryTypeHost;
+  return a.type != hipMemoryTypeUnregistered;
 }
 
 void stage_buffers(btpm_ctx* ctx) {
@@ -1530,7 +1530,7 @@ void par_memcpy(char* d, const char* s, size_t n) {
 
 void upload_staged(btpm_ctx* ctx, void* dst, const void* src, size_t bytes) {
   hipStream_t st = ctx->stream;
-  if (bytes < kStageUp || host_pinned(src)) {
+  if (bytes < kStageUp || dma_ready(src)) {
     if (bytes) HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st));
     HIPCHK(hipStreamSynchronize(st));
     return;
@@ -1554,7 +1554,7 @@ void upload_staged(btpm_ctx* ctx, void* dst, const void* src, size_t bytes) {
 
 void download_staged(btpm_ctx* ctx, void* dst, const void* src, size_t bytes) {
   hipStream_t st = ctx->stream;
-  if (bytes < kStageDown || host_pinned(dst)) {
+  if (bytes < kStageDown || dma_ready(dst)) {
     if (bytes) HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
     return;

@@ -467,6 +467,8 @@ __global__ __launch_bounds__(64, 2) void btpm_conduct_smooth_lin(
 #pragma unroll
     for (int k = 0; k < BTPM_BLK; ++k)
       gain[k] = reinterpret_cast<const float*>(opk + kGain)[k];
+    const float own_main = reinterpret_cast<const float*>(opk + kOwn)[0];
+    const float own_tail = reinterpret_cast<const float*>(opk + kOwn)[1];
     const gfloat* prof = (const gfloat*)S.prof;
     float u[NT][16];
 #pragma unroll
@@ -500,10 +502,11 @@ __global__ __launch_bounds__(64, 2) void btpm_conduct_smooth_lin(
       store_block(b, out);
       surface_in(u, w);
       if constexpr (FULL) {
-        linear_block<NT>(u, [&](int i) { return A[i]; });
+        if constexpr (NT == 4) linear_block_pairs(u, own_main, [&](int i) { return A[i]; });
+        else linear_block<NT>(u, own_main, [&](int i) { return A[i]; });
         surface_out(u, w);
       } else {
-        linear_block<NT>(u, [&](int i) { return (h8)op[(kFrags + i) * 64]; });
+        linear_block<NT>(u, own_tail, [&](int i) { return (h8)op[(kFrags + i) * 64]; });
       }
     };
     for (int b = 0; b + 1 < nb; ++b) block(b, std::true_type{});
@@ -1177,6 +1180,8 @@ __global__ __launch_bounds__((P * BTPM_NS + 63) / 64 * 64) void btpm_conduct_cra
 #pragma unroll
     for (int k = 0; k < BTPM_BLK; ++k)
       gain[k] = reinterpret_cast<const float*>(opk + kGain)[k];
+    const float own_main = reinterpret_cast<const float*>(opk + kOwn)[0];
+    const float own_tail = reinterpret_cast<const float*>(opk + kOwn)[1];
     const gfloat* prof = (const gfloat*)S.prof;
     float u[4][16];
 #pragma unroll
@@ -1250,24 +1255,15 @@ __global__ __launch_bounds__((P * BTPM_NS + 63) / 64 * 64) void btpm_conduct_cra
     for (int b = 0; b + 1 < nb; ++b) {
       block(b, std::true_type{});
       if constexpr (G::kOpLds) {
-        // two tiles at a time: a fragment read from LDS serves both
-        auto frag = [&](int i) { return lop[i * 64]; };
-        linear_block<2>(*reinterpret_cast<float (*)[2][16]>(&u[0]), frag);
-        asm volatile("" ::: "memory");
-        linear_block<2>(*reinterpret_cast<float (*)[2][16]>(&u[2]), frag);
+        linear_block_pairs(u, own_main, [&](int i) { return lop[i * 64]; });
       } else {
-        linear_block<4>(u, [&](int i) { return A[i]; });
+        linear_block<4>(u, own_main, [&](int i) { return A[i]; });
       }
       surface_out(u, w);
       __syncthreads();
     }
     block(nb - 1, std::false_type{});
-    {
-      auto frag = [&](int i) { return (h8)op[(kFrags + i) * 64]; };
-      linear_block<2>(*reinterpret_cast<float (*)[2][16]>(&u[0]), frag);
-      asm volatile("" ::: "memory");
-      linear_block<2>(*reinterpret_cast<float (*)[2][16]>(&u[2]), frag);
-    }
+    linear_block_pairs(u, own_tail, [&](int i) { return (h8)op[(kFrags + i) * 64]; });
 
 #pragma unroll
     for (int t = 0; t < 4; ++t) {

@@ -26,16 +26,30 @@
 // the 17-wide band of P^8 leaves the blocks (tile 0, chunk 1) and (tile 3,
 // chunk 0) empty: 6 of 8 blocks are stored and multiplied.
 //
-// Precision.  Operator and columns are split x = hi + lo in fp16 and
-// multiplied as lo hi + hi lo + hi hi with FP32 accumulation.  A column value
-// is FP32 (24 bits) and fp16 holds 11, so hi + lo (rounded to nearest) drops
-// at most one unit of the last FP32 place; the operator is scaled by 2^15 so
-// that its low halves stay normal numbers, and the rounding of its low halves
-// is carried along each row, so that constants stay constants to 2^-24 of an
-// ulp.  Columns are held multiplied by 2^15 (as the product leaves them).
-// Against FP64 over 24 to 60 rotations (r 0.03..0.497, inertias 30..2000) the
-// surface temperatures are within 6.3-7.5e-6 K rms, where eight FP32 steps
-// gave 6.8-7.7e-6 K: the rounding of the FP32 temperatures themselves.
+// Precision.  A node's own entry is nearly one when the FTCS number r is
+// small; what the product forms is the rest of the row,
+//     node' = c node + sum_j M_j entry_j,   M = P^8 - c I | H,
+// c the diagonal of an interior row in FP32, added by one FMA, so that the
+// product's rounding is that of the change over a block (about 16 r of the
+// node) and the node itself is rounded once.  M and the columns are split
+// x = hi + lo in fp16 and multiplied as hi hi + hi lo + lo hi with FP32
+// accumulation.  The matrix instruction cuts each of 8 products toward zero at
+// 2^-26 of the largest (by exponents) and its accumulator downward at 2^-26 of
+// them: one-sided, and what is one-sided adds up over the blocks.  So the large
+// products come first, and the hi halves of a row are whole multiples of 2^-15
+// of its largest power of two: products of columns alike in size are then not
+// cut at all.  M is scaled by 2^15 so that its low halves stay normal numbers.
+// The rounding of the low halves is made up on entries far from the node, whose
+// halves are finer: constants and linear profiles stay so (row sums to 4e-9,
+// first moments to 5e-7).  Columns are held multiplied by 2^15 (as the product
+// leaves them).  Errors against FP64 after 30 rotations, thermal inertias 20 to
+// 1000, in 1e-6 K rms of the surface / of all nodes, eight FP32 steps in
+// brackets:
+//   r 0.474   6.9 /  6.9  (7.2 /  6.9)      r 0.015   7.4 / 12.2  (7.8 / 12.0)
+//   r 0.126   7.1 /  7.7  (7.1 /  7.3)      r 0.0047  7.2 / 14.1  (7.7 / 14.8)
+//   r 0.030   7.4 / 10.6  (7.5 / 10.5)      r 0.0005  7.7 / 12.3  (8.7 / 13.0)
+// (P^8 whole in M, small products first: 40 to 60 for all nodes at r 0.03 to
+// 0.005.)
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -45,6 +59,7 @@
 
 namespace btpm_lin {
 
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
@@ -52,11 +67,13 @@ constexpr float kScale = 32768.0f;
 constexpr int kFrags = 12;              // 6 blocks x (hi, lo), 64 lanes x 8 halves each
 constexpr int kFrag = 64 * 8;           // halves per fragment
 // an operator in memory (halves): main[12], tail[12] (the last block's steps),
-// init[2] (base(1..8) of the first block from the nodes), then float g[8]
+// init[2] (base(1..8) of the first block from the nodes), then floats g[8] and
+// the c of main and tail
 constexpr int kTail = kFrags * kFrag;
 constexpr int kInit = 2 * kFrags * kFrag;
 constexpr int kGain = kInit + 2 * kFrag;
-static_assert(kGain + 16 <= BTPM_LIN_OP, "operator size");
+constexpr int kOwn = kGain + 2 * BTPM_BLK;
+static_assert(kOwn + 4 <= BTPM_LIN_OP, "operator size");
 
 // block b of the product: output tile and input chunk
 constexpr int kBlkTile[6] = {0, 1, 1, 2, 2, 3};
@@ -67,28 +84,32 @@ __device__ __forceinline__ int slot_node(int g, int q) {
   return q < 2 ? 0 : q < 4 ? 1 + 2 * g + (q - 2) : 9 + 16 * (q / 4 - 1) + 4 * g + (q & 3);
 }
 
-// fp16 hi / lo halves of 2^-15 x
-__device__ __forceinline__ void split2(float x, _Float16& hi, _Float16& lo) {
-  hi = (_Float16)fmaf(x, 1.0f / kScale, 0.0f);
-  lo = (_Float16)fmaf(x, 1.0f / kScale, -(float)hi);
+// fp16 hi / lo halves of 2^-15 x, two at a time: the empty asm keeps the hi
+// pair packed, so that the low halves are taken from it in place
+__device__ __forceinline__ void split2(float x, float y, h2& hi, h2& lo) {
+  hi = h2{(_Float16)fmaf(x, 1.0f / kScale, 0.0f), (_Float16)fmaf(y, 1.0f / kScale, 0.0f)};
+  asm volatile("" : "+v"(hi));
+  lo = h2{(_Float16)fmaf(x, 1.0f / kScale, -(float)hi.x),
+          (_Float16)fmaf(y, 1.0f / kScale, -(float)hi.y)};
+}
+// the 8 slots of input chunk h
+__device__ __forceinline__ void split_chunk(const float (&u)[16], int h, h8& hi, h8& lo) {
+  h2 a[4], b[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) split2(u[8 * h + 2 * j], u[8 * h + 2 * j + 1], a[j], b[j]);
+  hi = h8{a[0].x, a[0].y, a[1].x, a[1].y, a[2].x, a[2].y, a[3].x, a[3].y};
+  lo = h8{b[0].x, b[0].y, b[1].x, b[1].y, b[2].x, b[2].y, b[3].x, b[3].y};
 }
 
 // u <- operator u for NT tiles of 16 columns; frag(i) gives fragment i (block
-// i/2, hi then lo) of the lane
+// i/2, hi then lo) of the lane, own is c
 template <int NT, class Frag>
-__device__ __forceinline__ void linear_block(float (&u)[NT][16], Frag frag) {
+__device__ __forceinline__ void linear_block(float (&u)[NT][16], float own, Frag frag) {
   h8 bh[NT][2], bl[NT][2];
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        _Float16 a, b;
-        split2(u[t][8 * h + j], a, b);
-        bh[t][h][j] = a;
-        bl[t][h][j] = b;
-      }
+    for (int h = 0; h < 2; ++h) split_chunk(u[t], h, bh[t][h], bl[t][h]);
 #pragma unroll
   for (int ot = 0; ot < 4; ++ot) {
     f4 acc[NT];
@@ -101,7 +122,6 @@ __device__ __forceinline__ void linear_block(float (&u)[NT][16], Frag frag) {
         ahi[kBlkChunk[b]] = frag(2 * b);
         alo[kBlkChunk[b]] = frag(2 * b + 1);
       }
-    // small products first
 #pragma unroll
     for (int p = 0; p < 3; ++p)
 #pragma unroll
@@ -110,15 +130,25 @@ __device__ __forceinline__ void linear_block(float (&u)[NT][16], Frag frag) {
 #pragma unroll
           for (int t = 0; t < NT; ++t) {
             const int h = kBlkChunk[b];
-            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(p == 0 ? alo[h] : ahi[h],
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(p == 2 ? alo[h] : ahi[h],
                                                             p == 1 ? bl[t][h] : bh[t][h], acc[t],
                                                             0, 0, 0);
           }
+    // (tile 0, i < 2: a surface slot)
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) u[t][4 * ot + i] = acc[t][i];
+      for (int i = 0; i < 4; ++i)
+        u[t][4 * ot + i] = ot == 0 && i < 2 ? acc[t][i] : fmaf(own, u[t][4 * ot + i], acc[t][i]);
   }
+}
+
+// four tiles, two at a time: half the registers for the split columns
+template <class Frag>
+__device__ __forceinline__ void linear_block_pairs(float (&u)[4][16], float own, Frag frag) {
+  linear_block<2>(*reinterpret_cast<float (*)[2][16]>(&u[0]), own, frag);
+  asm volatile("" ::: "memory");
+  linear_block<2>(*reinterpret_cast<float (*)[2][16]>(&u[2]), own, frag);
 }
 
 // base(1..8) of a rotation's first block from the nodes (surface slots zero)
@@ -127,17 +157,11 @@ __device__ __forceinline__ void linear_init(float (&u)[NT][16], h8 ahi, h8 alo) 
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     h8 bh, bl;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      _Float16 a, b;
-      split2(u[t][j], a, b);
-      bh[j] = a;
-      bl[j] = b;
-    }
+    split_chunk(u[t], 0, bh, bl);
     f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bh, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bl, acc, 0, 0, 0);
     acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bh, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bl, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bh, acc, 0, 0, 0);
     u[t][0] = acc[0];
     u[t][1] = acc[1];
   }

@@ -59,25 +59,68 @@ void respond(double r, int steps, bool responses, double (&out)[L][L]) {
   }
 }
 
-// hi and lo of every entry times 2^15, the rounding of the low halves carried
-// along the row from its largest entry to its smallest
+// takes the diagonal c of an interior row off the node rows; returns it
+float take_own(double (&m)[L][L]) {
+  const float c = (float)m[N / 2][N / 2];
+  for (int i = 0; i < N; ++i) m[i][i] -= (double)c;
+  return c;
+}
+
+// hi and lo of every entry times 2^15.  The hi halves of a row are whole
+// multiples of 2^-15 of its largest power of two.  The error of a row's sum and
+// of its first moment about the row's node (entries at their nodes, surface
+// values at node 0), left by rounding the low halves, are then made up on two
+// entries at a distance d to either side, d = 1..8: those of the far entries,
+// which are small and so are their units, are exact enough.  What is left of
+// the sum goes to the row's smallest entry.
 void split_rows(const double (&m)[L][L], _Float16 (&hi)[L][L], _Float16 (&lo)[L][L]) {
   std::memset(hi, 0, sizeof hi);
   std::memset(lo, 0, sizeof lo);
+  auto pos = [](int j) { return j < N ? j + 1 : 0; };
   for (int i = 0; i < L; ++i) {
-    int by[L], n = 0;
-    for (int j = 0; j < L; ++j)
-      if (m[i][j] != 0.0) by[n++] = j;
-    std::sort(by, by + n, [&](int a, int b) { return std::fabs(m[i][a]) > std::fabs(m[i][b]); });
-    double carry = 0.0;
-    for (int k = 0; k < n; ++k) {
-      const int j = by[k];
-      const double x = m[i][j] * btpm_lin::kScale;
-      hi[i][j] = (_Float16)x;
-      const double w = x - (double)hi[i][j] + carry;
-      lo[i][j] = (_Float16)w;
-      carry = w - (double)lo[i][j];
+    double top = 0.0;
+    int least = -1;
+    for (int j = 0; j < L; ++j) {
+      const double a = std::fabs(m[i][j]);
+      top = std::fmax(top, a);
+      if (a > 0.0 && (least < 0 || a < std::fabs(m[i][least]))) least = j;
     }
+    if (least < 0) continue;
+    int e;
+    std::frexp(top * btpm_lin::kScale, &e);
+    const double unit = std::ldexp(1.0, e - 15);
+    for (int j = 0; j < L; ++j) {
+      if (m[i][j] == 0.0) continue;
+      const double x = m[i][j] * btpm_lin::kScale;
+      double h = (double)(_Float16)x;
+      if (std::fabs(h) < 2048.0 * unit) h = (double)(_Float16)(std::rint(x / unit) * unit);
+      hi[i][j] = (_Float16)h;
+      lo[i][j] = (_Float16)(x - h);
+    }
+    const int at = i < N ? i + 1 : 1;
+    double sum = 0.0, mom = 0.0;
+    for (int j = 0; j < L; ++j) {
+      if (m[i][j] == 0.0) continue;
+      const double err = (double)hi[i][j] + (double)lo[i][j] - m[i][j] * btpm_lin::kScale;
+      sum += err;
+      mom += err * (pos(j) - at);
+    }
+    auto change = [&](int j, double by) {
+      const double was = (double)lo[i][j];
+      lo[i][j] = (_Float16)(was + by);
+      const double d = (double)lo[i][j] - was;
+      sum += d;
+      mom += d * (pos(j) - at);
+    };
+    for (int d = 1; d <= B; ++d) {
+      const int p = at > d ? at - d - 1 : N, q = std::min(at + d, N) - 1;
+      if (m[i][p] == 0.0 || m[i][q] == 0.0 || pos(p) == pos(q)) continue;
+      const double dp = pos(p) - at, dq = pos(q) - at;
+      const double b = (sum * dp - mom) / (dq - dp), a = -sum - b;
+      change(p, a);
+      change(q, b);
+    }
+    change(least, -sum);
   }
 }
 
@@ -99,11 +142,14 @@ void linear_operator(float rf, int ntau, _Float16* op) {
   static thread_local double m[L][L];
   static thread_local _Float16 hi[L][L], lo[L][L];
   std::fill(op, op + BTPM_LIN_OP, (_Float16)0.0f);
+  float own[2];
   respond(r, B, true, m);
+  own[0] = take_own(m);
   split_rows(m, hi, lo);
   for (int b = 0; b < 6; ++b) pack(hi, lo, btpm_lin::kBlkTile[b], btpm_lin::kBlkChunk[b], op + 2 * b * btpm_lin::kFrag);
   // the last block's steps: nodes only
   respond(r, ntau - (nblocks(ntau) - 1) * B, false, m);
+  own[1] = take_own(m);
   split_rows(m, hi, lo);
   for (int b = 0; b < 6; ++b)
     pack(hi, lo, btpm_lin::kBlkTile[b], btpm_lin::kBlkChunk[b], op + btpm_lin::kTail + 2 * b * btpm_lin::kFrag);
@@ -122,5 +168,6 @@ void linear_operator(float rf, int ntau, _Float16* op) {
     g[k] = (float)u[0][0];
   }
   std::memcpy(op + btpm_lin::kGain, g, sizeof g);
+  std::memcpy(op + btpm_lin::kOwn, own, sizeof own);
 }
 }  // namespace btpm

@@ -31,7 +31,6 @@
 #include "btpm_device.h"
 #include "linear_block.h"
 
-typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 // Pointers read from the set descriptor are generic; casting them to the
 // global address space lets the compiler emit global (not flat) memory ops,
@@ -551,8 +550,8 @@ template __global__ void btpm_conduct_smooth_lin<4>(const btpm_tile*, const btpm
 // the workgroup evaluates the crater self-heating of all its craters for the
 // 8 steps at once as one MFMA product
 //     Q[j][n] = sum_i VF(j->i) E[i][n],   n = (crater, step in block)
-// with M = 100 (padded 112), K = 100 (padded 112), N = 80, using
-// v_mfma_f32_16x16x16_f16 and the three-product split
+// with M = 100 (padded 112), K = 100 (padded 128), N = 80, using
+// v_mfma_f32_16x16x32_f16 and the three-product split
 //     VF E ~ VFhi Ehi + VFhi Elo + VFlo Ehi   (FP32 accumulation),
 // where x_hi = fp16(x) and x_lo = fp16(x - x_hi).  VF is stored pre-scaled by
 // 2^s (max entry in [0.5, 1)) so its low halves stay normal fp16 numbers;
@@ -581,9 +580,12 @@ constexpr int kNT = kNP / 16;      // 5 N tiles
 //
 // The phase is bound by the latency of its LDS fragment reads, so a wave
 // computes a strip of one m tile and 3 (or 2) n tiles, reading each A fragment
-// once per K chunk for the whole strip; K runs as 3 chunks of 32
-// (v_mfma_f32_16x16x32_f16, 16-byte fragment reads) plus the tail k = 96..99
-// as one 16x16x16 chunk in which only the 16 lanes holding sub-facets read.
+// once per K chunk for the whole strip; K runs as 4 chunks of 32
+// (v_mfma_f32_16x16x32_f16, 16-byte fragment reads), the last with the tail
+// k = 96..99 in its first slots and zeros in the others.  One instruction
+// shape throughout: a 16x16x16 instruction that adds to what a 16x16x32 has
+// just left there was seen to give wrong rows 4g, 4g + 1, and what keeps the
+// two far enough apart is then up to the schedule.
 // The 14 strips (7 m tiles x {n 0-2, n 3-4}) sit on the waves so that each
 // SIMD (waves s, s+4, s+8, s+12) carries at most 9 of the 35 output tiles;
 // waves 12 and 13 have none.  Within a lane, fragment slot j of A and of B
@@ -591,12 +593,17 @@ constexpr int kNT = kNP / 16;      // 5 N tiles
 //
 // One K chunk of 32 (v_mfma_f32_16x16x32_f16): lane l supplies
 // A[m = l%16][k = 8(l/16) .. +7] and B[k = 8(l/16) .. +7][n = l%16].
-// The low halves lie AH (of A) and BH (of B) halves behind the high ones.
+// The low halves lie AH (of A) and BH (of B) halves behind the high ones; A
+// counts as zero in lanes without `use`.
 template <int NNT, int AH, int BH>
 __device__ __forceinline__ void strip_chunk32(const _Float16* lds_a, const _Float16* lds_b, int am,
-                                              int k0, int nt0, int r, float4_t (&acc)[NNT]) {
-  const half8_t ahi = *reinterpret_cast<const half8_t*>(&lds_a[am * kLdsK + k0]);
-  const half8_t alo = *reinterpret_cast<const half8_t*>(&lds_a[AH + am * kLdsK + k0]);
+                                              int k0, int nt0, int r, bool use,
+                                              float4_t (&acc)[NNT]) {
+  const half8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};
+  half8_t ahi = *reinterpret_cast<const half8_t*>(&lds_a[am * kLdsK + k0]);
+  half8_t alo = *reinterpret_cast<const half8_t*>(&lds_a[AH + am * kLdsK + k0]);
+  ahi = use ? ahi : zero;
+  alo = use ? alo : zero;
 #pragma unroll
   for (int t = 0; t < NNT; ++t) {
     const int bn = (nt0 + t) * 16 + r;
@@ -615,40 +622,21 @@ __device__ __forceinline__ void product_strip(const _Float16* lds_a, const _Floa
                                               float* lds_q, int mt, int nt0, int lane,
                                               float unscale) {
   constexpr int kFull = BTPM_NS / 32 * 32;  // 96: sub-facets in full chunks of 32
-  static_assert(BTPM_NS - kFull == 4 && kKP >= kFull + 16, "one partial K chunk of 4");
+  static_assert(BTPM_NS - kFull == 4 && kLdsK == kFull + 8, "one partial K chunk of 4");
   float4_t acc[NNT];
 #pragma unroll
   for (int t = 0; t < NNT; ++t) acc[t] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
   const int r = lane & 15;
   const int g = lane >> 4;
   const int am = mt * 16 + r;
+  // the tail k = 96..99 as a fourth chunk of 32 whose other slots are zero: A
+  // in the lanes past the first 16 (B is read by all, so a NaN there is one of
+  // the column's own), and k = 100..103 are zero in both
 #pragma unroll 1
-  for (int kt = 0; kt < kFull / 32; ++kt)
-    strip_chunk32<NNT, AH, BH>(lds_a, lds_b, am, kt * 32 + 8 * g, nt0, r, acc);
-  // the tail k = 96..99 as one v_mfma_f32_16x16x16f16 chunk (k = 4(l/16)..+3):
-  // only lanes 0-15 hold sub-facets, the others contribute zero operands
-  // instead of reading the zero padding
-  {
-    const half4_t zero = {0, 0, 0, 0};
-    half4_t ahi = zero, alo = zero, bhi[NNT], blo[NNT];
-#pragma unroll
-    for (int t = 0; t < NNT; ++t) bhi[t] = blo[t] = zero;
-    if (g == 0) {
-      ahi = *reinterpret_cast<const half4_t*>(&lds_a[am * kLdsK + kFull]);
-      alo = *reinterpret_cast<const half4_t*>(&lds_a[AH + am * kLdsK + kFull]);
-#pragma unroll
-      for (int t = 0; t < NNT; ++t) {
-        const int bn = (nt0 + t) * 16 + r;
-        bhi[t] = *reinterpret_cast<const half4_t*>(&lds_b[bn * kLdsK + kFull]);
-        blo[t] = *reinterpret_cast<const half4_t*>(&lds_b[BH + bn * kLdsK + kFull]);
-      }
-    }
-#pragma unroll
-    for (int t = 0; t < NNT; ++t) {
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x16f16(alo, bhi[t], acc[t], 0, 0, 0);
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x16f16(ahi, blo[t], acc[t], 0, 0, 0);
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x16f16(ahi, bhi[t], acc[t], 0, 0, 0);
-    }
+  for (int kt = 0; kt <= kFull / 32; ++kt) {
+    const bool tail = kt == kFull / 32;
+    strip_chunk32<NNT, AH, BH>(lds_a, lds_b, am, tail ? kFull : kt * 32 + 8 * g, nt0, r,
+                               !tail || g == 0, acc);
   }
   const int m0 = mt * 16 + 4 * g;  // 4 receiving sub-facets m0 .. m0 + 3
   if (m0 < BTPM_NS) {
@@ -950,7 +938,7 @@ extern "C" __global__ __launch_bounds__(BTPM_CRATER_THREADS) void btpm_conduct_c
 // the balance's dependent FP64 chain), and the emission of block b + 2 is
 // split after them: E and Q are double buffered and a block has one barrier.
 // The fragments that do not change (the wave's m tiles of VF^T, at P = 2
-// the operator too) stay in registers for the whole rotation.P = 5
+// the operator too) stay in registers for the whole rotation.  P = 5
 // puts 98 % of its lanes to work, two waves to a SIMD; P = 2 spreads few
 // craters over more CUs, one wave to a SIMD.  A 650-step rotation of 80
 // craters takes 232 us at P = 2, 345 us at P = 5 (one crater a workgroup: 259
@@ -975,9 +963,7 @@ struct CraterGroup {
 };
 
 // A fragments of one m tile of VF^T: three K chunks of 32 and the tail 96..99
-// as a fourth whose other slots are zero.  (A 16x16x16 product for the tail
-// right behind the 16x16x32 ones it adds to gave wrong rows 4g, 4g + 1: the
-// two have different pass counts, so they are not chained here.)
+// as a fourth whose other slots are zero, as in product_strip.
 struct VfFrag {
   half8_t hi[4], lo[4];
 };

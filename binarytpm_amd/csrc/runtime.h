@@ -194,8 +194,8 @@ namespace btpm {
 // Host-to-device copy of a large pageable buffer, complete on return: slices
 // are copied by host threads into one of the context's two pinned staging
 // buffers while the DMA of the other slice runs on the context's stream.
-// Small copies and pinned buffers go straight to hipMemcpyAsync.  Caller holds
-// ctx->mu.
+// Small copies, pinned buffers, and all where no memory can be pinned, go
+// straight to hipMemcpyAsync.  Caller holds ctx->mu.  (staging.hip)
 void upload_staged(btpm_ctx* ctx, void* dst, const void* src, size_t bytes);
 // The device-to-host counterpart: the DMA of the next slice runs while host
 // threads copy the previous one out of its pinned buffer.

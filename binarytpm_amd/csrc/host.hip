@@ -717,37 +717,29 @@ struct Sched {
     return c;
   }
   // The operator's kernels (16, 32 or 64 columns per wave) share a launch, and
-  // what a width costs turns on how many waves all their sets make together.
-  // Measured per 650-step rotation at 16 / 32 / 64: 5120 columns 101 / 121 /
-  // 163 us, 20480 columns 123 / 125 / 165 us, 40960 columns 156 / 154 / 170 us,
-  // 81920 columns 222 / 206 / 217 us: 16 up to kLinCols columns, 32 beyond.
-  // A trial runs in the first rotations, whose extra Newton iterations favour
-  // wide waves, so another width must be kLinMargin cheaper there.
-  static constexpr long long kLinCols = 20480;
+  // what a width costs turns on how many waves all their sets make together
+  // (smooth_lin_width).  A trial runs in the first rotations, whose extra Newton
+  // iterations favour wide waves, so another width must be kLinMargin cheaper
+  // there.
   static constexpr double kLinMargin = 0.10;
   TuneKey smooth_key(const SetHost* S) const {
     const long long c = log2_class(S->d.ncols);
-    return S->d.op ? TuneKey{2, c | (linear_cols() > kLinCols ? 64 : 0)} : TuneKey{0, c};
+    return S->d.op ? TuneKey{2, c | (smooth_lin_width(linear_cols(), ctx->cus) > 16 ? 64 : 0)} : TuneKey{0, c};
   }
   int smooth_default(const SetHost* S) const {
-    return S->d.op ? (linear_cols() > kLinCols ? 32 : 16) : BTPM_SMOOTH_WG;
+    return S->d.op ? smooth_lin_width(linear_cols(), ctx->cus) : BTPM_SMOOTH_WG;
   }
   std::vector<int> smooth_candidates(const SetHost* S) const {
     if (!S->d.op) return {256, 128, 64};
     return smooth_default(S) == 16 ? std::vector<int>{16, 32, 64} : std::vector<int>{32, 16, 64};
   }
-  // Craters per workgroup of the operator's crater conduction, for all such
-  // sets of a rotation together: 2 while every workgroup has a CU to itself
-  // (512 craters: 290 us a rotation against 399 us with 5), else 5 (640
-  // craters: 415 us against 534 us with 2, which then takes two rounds).
-  static constexpr long long kPairCraters = 512;
   int crater_width() const {
     long long n = 0;
     for (auto& kv : slots) {
       const SetHost* S = kv.second.second;
       if (S->d.kind == BTPM_SET_CRATER && S->d.op) n += ctx->h_status[S->slot].norder;
     }
-    return n <= kPairCraters ? 2 : 5;
+    return crater_lin_width(n, ctx->cus);
   }
   static TuneKey heat_key(const btpm_shape* sh) {
     return {1, (log2_class(sh->nnz) << 40) | (log2_class(sh->nf) << 24) | sh->nb};
@@ -1512,6 +1504,7 @@ int btpm_ctx_create(int device, btpm_ctx** out) {
   noalloc_setup(device);  // this device's scratch of the allocation-free entry point
   auto c = std::make_unique<btpm_ctx>();
   c->device = device;
+  HIPCHK(hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, device));
   HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
   HIPCHK(hipMalloc(&c->d_sets, sizeof(btpm_set_dev) * kMaxSets));
   HIPCHK(hipMalloc(&c->d_status, sizeof(btpm_status_dev) * kMaxSets));

@@ -89,6 +89,18 @@ inline unsigned grid_stride(size_t n, unsigned b) {
   return (unsigned)(g < 16384 ? (g > 0 ? g : 1) : 16384);
 }
 
+// Columns per wave of the operator's smooth conduction (16, 32 or 64), all sets
+// of a launch together.  Measured on 256 CUs per 650-step rotation at 16 / 32 /
+// 64: 5120 columns 100 / 120 / 162 us, 20480 columns 122 / 125 / 165 us, 40960
+// columns 156 / 152 / 170 us, 81920 columns 222 / 204 / 217 us: 16 while that
+// is at most five waves per CU, 32 beyond.
+inline int smooth_lin_width(long long columns, int cus) { return columns <= 80LL * cus ? 16 : 32; }
+// Craters per workgroup of the operator's crater conduction, all sets of a
+// rotation together: 2 while every workgroup has a CU to itself (512 craters on
+// 256 CUs: 290 us a rotation against 399 us with 5), else 5 (640 craters: 415 us
+// against 534 us with 2, which then takes two rounds).
+inline int crater_lin_width(long long craters, int cus) { return craters <= 2LL * cus ? 2 : 5; }
+
 // device buffer owned by RAII
 // Device memory cache.  Blocks released by DBuf stay cached per device and
 // are handed out again best-fit (capacity within 1.25x of the request):
@@ -170,6 +182,7 @@ float vf_tiles(const float* vf, std::vector<_Float16>& a);
 // one device: its stream and the resident-set tables of the scheduler
 struct btpm_ctx {
   int device = 0;
+  int cus = 0;  // compute units
   hipStream_t stream = nullptr;
   btpm_set_dev* d_sets = nullptr;
   btpm_status_dev* d_status = nullptr;

@@ -638,13 +638,13 @@ struct Sched {
   std::vector<TileList> crater_lists;
   static constexpr int kLinear = 1 << 16;
   // columns of the resident smooth sets on the 8-step operator
-  long long linear_cols() const {
-    long long cols = 0;
+  long long lin_cols = 0;
+  void count_lin_cols() {
+    lin_cols = 0;
     for (auto& kv : slots) {
       const SetHost* S = kv.second.second;
-      if (S->d.kind == BTPM_SET_SMOOTH && S->d.op) cols += S->d.ncols;
+      if (S->d.kind == BTPM_SET_SMOOTH && S->d.op) lin_cols += S->d.ncols;
     }
-    return cols;
   }
   // smooth sets with facet self-heating, grouped by shape: one tiled SpMM
   // launch per group per rotation
@@ -685,7 +685,8 @@ struct Sched {
   // Tile choices per size class, measured on the device:
   //   kind 0: smooth conduction columns per workgroup {256, 128, 64}, per
   //           column-count class (ceil log2 of the set's columns); kind 2: of
-  //           the 8-step operator's kernels {16, 32, 64};
+  //           the 8-step operator's kernels {16, 32, 64}, per class of the
+  //           columns of all their sets;
   //   kind 1: facet self-heating kernel {time-lane (0), per-chunk CSR or ELL
   //           64, ELL 32, receiver-grouped} as the shape's layouts allow, per
   //           (log2 nnz, log2 facets, step blocks) class.
@@ -717,17 +718,20 @@ struct Sched {
     return c;
   }
   // The operator's kernels (16, 32 or 64 columns per wave) share a launch, and
-  // what a width costs turns on how many waves all their sets make together
-  // (smooth_lin_width).  A trial runs in the first rotations, whose extra Newton
-  // iterations favour wide waves, so another width must be kLinMargin cheaper
-  // there.
+  // what a width costs turns on how many waves all their sets make together:
+  // they are one class per factor of 4 in their columns, counted from where the
+  // untuned width changes (smooth_lin_width).  A trial runs in the first
+  // rotations, whose extra Newton iterations favour wide waves, so another
+  // width must be kLinMargin cheaper there.
   static constexpr double kLinMargin = 0.10;
   TuneKey smooth_key(const SetHost* S) const {
-    const long long c = log2_class(S->d.ncols);
-    return S->d.op ? TuneKey{2, c | (smooth_lin_width(linear_cols(), ctx->cus) > 16 ? 64 : 0)} : TuneKey{0, c};
+    if (!S->d.op) return {0, log2_class(S->d.ncols)};
+    long long load = 0;
+    for (long long n = lin_cols; smooth_lin_width(n, ctx->cus) > 16; n /= 4) ++load;
+    return {2, load};
   }
   int smooth_default(const SetHost* S) const {
-    return S->d.op ? smooth_lin_width(linear_cols(), ctx->cus) : BTPM_SMOOTH_WG;
+    return S->d.op ? smooth_lin_width(lin_cols, ctx->cus) : BTPM_SMOOTH_WG;
   }
   std::vector<int> smooth_candidates(const SetHost* S) const {
     if (!S->d.op) return {256, 128, 64};
@@ -1022,6 +1026,7 @@ struct Sched {
   }
 
   void rebuild_lists() {
+    count_lin_cols();
     // tuning: classes present without a decision get a trial; a trial whose
     // sets have all left is dropped (it restarts if the class returns)
     std::map<btpm_shape*, std::vector<int>> by_shape;

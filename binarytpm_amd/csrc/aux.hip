@@ -720,7 +720,8 @@ extern "C" __global__ __launch_bounds__(256) void btpm_crater_scatter(
 #pragma unroll
       for (int t = 0; t < 2; ++t) own[m][t] = sp[m][t];
   }
-  // out through the buffer that the last sweep did not read
+  // out through the other buffer: the last sweep of the fixed point read it, and
+  // the barrier behind its put() lies between (else it was never read)
   put(il[cur ^ 1], 1.0f);
   __syncthreads();
   const int ncols = nfac * NS;

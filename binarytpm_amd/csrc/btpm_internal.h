@@ -101,7 +101,7 @@ struct btpm_set_dev {
   float* qext;        // [nb][ncols][BLK] total flux incl. facet self-heating (or null)
   float* emis;        // [ncols][nb*BLK] esia T^4 for the next rotation (or null),
                       // facet-major for the self-heating SpMM's coalesced reads
-  const void* op;     // 8-step conduction operator of the set's FTCS number (linear_block.h)
+  const void* op;     // 8-step conduction operators, one per class (linear_block.h; null: none)
   const float* vfA;   // crater: fp16 hi/lo view-factor tiles (see crater kernel)
   // status, written by the kernels
   int* tile_active;   // [ntiles] active groups after this rotation's test

@@ -88,7 +88,7 @@ __device__ __forceinline__ int slot_node(int g, int q) {
 // pair packed, so that the low halves are taken from it in place
 __device__ __forceinline__ void split2(float x, float y, h2& hi, h2& lo) {
   hi = h2{(_Float16)fmaf(x, 1.0f / kScale, 0.0f), (_Float16)fmaf(y, 1.0f / kScale, 0.0f)};
-  asm volatile("" : "+v"(hi));
+  asm("" : "+v"(hi));
   lo = h2{(_Float16)fmaf(x, 1.0f / kScale, -(float)hi.x),
           (_Float16)fmaf(y, 1.0f / kScale, -(float)hi.y)};
 }

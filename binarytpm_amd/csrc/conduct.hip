@@ -940,11 +940,11 @@ extern "C" __global__ __launch_bounds__(BTPM_CRATER_THREADS) void btpm_conduct_c
 // The fragments that do not change (the wave's m tiles of VF^T, at P = 2
 // the operator too) stay in registers for the whole rotation.  P = 5
 // puts 98 % of its lanes to work, two waves to a SIMD; P = 2 spreads few
-// craters over more CUs, one wave to a SIMD.  A 650-step rotation of 80
-// craters takes 232 us at P = 2, 345 us at P = 5 (one crater a workgroup: 259
-// us, four m tiles per wave), where ten craters a workgroup with the steps on
-// the vector ALUs took 663 us; 512 craters 290 / 399 us, 640 craters 534 /
-// 415 us, 5120 craters 1.69 / 1.17 ms (1.19 ms on the vector ALUs).
+// craters over more CUs, one wave to a SIMD.  A 650-step rotation, none frozen,
+// at P = 2 / 5 and with ten craters a workgroup and the steps on the vector
+// ALUs: 80 craters 267 / 389 / 718 us, 512 craters 292 / 403 / 756 us, 640
+// craters 525 / 411 / 744 us, 5120 craters 2.58 / 1.69 / 1.73 ms: on a full chip
+// the operator only holds what the vector ALUs reach.
 // ---------------------------------------------------------------------------
 namespace {
 template <int P>

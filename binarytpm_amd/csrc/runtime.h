@@ -90,15 +90,17 @@ inline unsigned grid_stride(size_t n, unsigned b) {
 }
 
 // Columns per wave of the operator's smooth conduction (16, 32 or 64), all sets
-// of a launch together.  Measured on 256 CUs per 650-step rotation at 16 / 32 /
-// 64: 5120 columns 100 / 120 / 162 us, 20480 columns 122 / 125 / 165 us, 40960
-// columns 156 / 152 / 170 us, 81920 columns 222 / 204 / 217 us: 16 while that
-// is at most five waves per CU, 32 beyond.
+// of a launch together.  Measured on 256 CUs, mean 650-step rotation of a solve
+// (its columns freeze one by one) at 16 / 32 / 64: 5120 columns 100 / 118 / 161
+// us, 20480 columns 123 / 124 / 163 us, 40960 columns 155 / 152 / 168 us, 81920
+// columns 220 / 204 / 212 us: 16 while that is at most five waves per CU, 32
+// beyond.  (While none has frozen: 5120 columns 148 / 159 / 199 us, 20480
+// columns 194 / 170 / 210 us, 81920 columns 387 / 341 / 315 us.)
 inline int smooth_lin_width(long long columns, int cus) { return columns <= 80LL * cus ? 16 : 32; }
 // Craters per workgroup of the operator's crater conduction, all sets of a
 // rotation together: 2 while every workgroup has a CU to itself (512 craters on
-// 256 CUs: 290 us a rotation against 399 us with 5), else 5 (640 craters: 415 us
-// against 534 us with 2, which then takes two rounds).
+// 256 CUs: 292 us a rotation against 403 us with 5), else 5 (640 craters: 411 us
+// against 525 us with 2, which then takes two rounds).
 inline int crater_lin_width(long long craters, int cus) { return craters <= 2LL * cus ? 2 : 5; }
 
 // device buffer owned by RAII

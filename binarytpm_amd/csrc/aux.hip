@@ -120,40 +120,45 @@ extern "C" __global__ __launch_bounds__(256) void btpm_init_smooth(btpm_set_dev 
   constexpr int kCols = 8, kParts = 32;
   __shared__ double part[kParts][kCols];
   const int lc = threadIdx.x % kCols, p = threadIdx.x / kCols;
-  const int c = min(blockIdx.x * kCols + lc, (unsigned)S.ncols - 1u);
-  const bool ok = blockIdx.x * kCols + lc < (unsigned)S.ncols;
-  double sum = 0.0;
-  for (int b = p; b < S.nb; b += kParts) {
-    const float4* v = reinterpret_cast<const float4*>(S.src + ((size_t)b * S.ncols + c) * BTPM_BLK);
-    const float4 x = v[0], y = v[1];
-    const float e[BTPM_BLK] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
-    const int kend = min(BTPM_BLK, S.ntau - b * BTPM_BLK);
+  // (32 lanes a column: 2^27 columns would be more work-items than a launch has)
+  for (unsigned c0 = blockIdx.x * kCols; c0 < (unsigned)S.ncols; c0 += gridDim.x * kCols) {
+    const bool ok = c0 + lc < (unsigned)S.ncols;
+    const size_t c = ok ? c0 + lc : (unsigned)S.ncols - 1u;
+    double sum = 0.0;
+    for (int b = p; b < S.nb; b += kParts) {
+      const float4* v =
+          reinterpret_cast<const float4*>(S.src + ((size_t)b * S.ncols + c) * BTPM_BLK);
+      const float4 x = v[0], y = v[1];
+      const float e[BTPM_BLK] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+      const int kend = min(BTPM_BLK, S.ntau - b * BTPM_BLK);
 #pragma unroll
-    for (int k = 0; k < BTPM_BLK; ++k)
-      if (k < kend) sum += (double)e[k];
-  }
-  part[p][lc] = sum;
-  __syncthreads();
-  sum = 0.0;
-  for (int q = 0; q < kParts; ++q) sum += part[q][lc];
-  if (!ok) return;
-  const float t = (float)pow(sum / S.ntau / (double)S.es, 0.25);
-  const float4 t4 = make_float4(t, t, t, t);
-  const float e = S.esia * t * t * t * t;
-  const float4 e4 = make_float4(e, e, e, e);
-  for (int i = p; i < BTPM_PSTRIDE / 4; i += kParts)
-    reinterpret_cast<float4*>(S.prof + (size_t)c * BTPM_PSTRIDE)[i] = t4;
-  for (int b = p; b < S.nb; b += kParts) {
-    float4* v = reinterpret_cast<float4*>(S.T + ((size_t)b * S.ncols + c) * BTPM_BLK);
-    v[0] = t4;
-    v[1] = t4;
-  }
-  if (S.emis)  // facet-major [c][nb*BLK]
-    for (int i = p; i < S.nb * (BTPM_BLK / 4); i += kParts)
-      reinterpret_cast<float4*>(S.emis + (size_t)c * S.nb * BTPM_BLK)[i] = e4;
-  if (p == 0) {
-    S.frozen[c] = 0;
-    S.dmax[c] = 0.0f;
+      for (int k = 0; k < BTPM_BLK; ++k)
+        if (k < kend) sum += (double)e[k];
+    }
+    part[p][lc] = sum;
+    __syncthreads();
+    sum = 0.0;
+    for (int q = 0; q < kParts; ++q) sum += part[q][lc];
+    __syncthreads();  // read before the next columns' sums
+    if (!ok) continue;
+    const float t = (float)pow(sum / S.ntau / (double)S.es, 0.25);
+    const float4 t4 = make_float4(t, t, t, t);
+    const float e = S.esia * t * t * t * t;
+    const float4 e4 = make_float4(e, e, e, e);
+    for (int i = p; i < BTPM_PSTRIDE / 4; i += kParts)
+      reinterpret_cast<float4*>(S.prof + c * BTPM_PSTRIDE)[i] = t4;
+    for (int b = p; b < S.nb; b += kParts) {
+      float4* v = reinterpret_cast<float4*>(S.T + ((size_t)b * S.ncols + c) * BTPM_BLK);
+      v[0] = t4;
+      v[1] = t4;
+    }
+    if (S.emis)  // facet-major [c][nb*BLK]
+      for (int i = p; i < S.nb * (BTPM_BLK / 4); i += kParts)
+        reinterpret_cast<float4*>(S.emis + c * S.nb * BTPM_BLK)[i] = e4;
+    if (p == 0) {
+      S.frozen[c] = 0;
+      S.dmax[c] = 0.0f;
+    }
   }
 }
 

@@ -490,7 +490,7 @@ void build_smooth(btpm_solve* s, hipStream_t st) {
                           hipMemcpyDeviceToDevice, st));
     hipLaunchKernelGGL(btpm_warm_smooth, dim3(grid1(d.ncols, 256)), dim3(256), 0, st, d);
   } else {
-    hipLaunchKernelGGL(btpm_init_smooth, dim3(grid1(d.ncols, 8)), dim3(256), 0, st, d);
+    hipLaunchKernelGGL(btpm_init_smooth, dim3(grid_stride(d.ncols, 8)), dim3(256), 0, st, d);
   }
   HIPCHK(hipGetLastError());
   s->smooth = std::move(S);
